@@ -55,8 +55,11 @@ class MpnnGraph {
   const int32_t* idx_;
   hipStream_t s_;
   int32_t *row_ = nullptr, *rev_ = nullptr;
-  double *scale_ = nullptr, *feat_ = nullptr, *pre1_ = nullptr, *node_ = nullptr, *pre2_ = nullptr, *out_ = nullptr;
-  double *go_ = nullptr, *dz_ = nullptr, *dnode_ = nullptr, *dpre1_ = nullptr, *dpre2_ = nullptr;
+  // pq_: W2b n_i + b2 and W2c n_i of every node; sr_: the sums of dL/dpre2 over
+  // the blocks of every node's row and over their reverses
+  double *scale_ = nullptr, *feat_ = nullptr, *pre1_ = nullptr, *node_ = nullptr, *pq_ = nullptr, *pre2_ = nullptr,
+         *out_ = nullptr;
+  double *go_ = nullptr, *d2_ = nullptr, *dm_ = nullptr, *sr_ = nullptr, *dnode_ = nullptr, *part_ = nullptr;
 };
 
 }  // namespace rf

@@ -68,6 +68,32 @@ def test_loss_and_gradient_match_oracle(rf):
         assert abs(fd - g[k]) <= 1e-5 * gmax, (k, fd, g[k])
 
 
+@pytest.mark.parametrize("nx,nvec,nu", [(1, 1, 1), (2, 3, 2), (3, 8, 1), (5, 1, 3), (6, 300, 2)])
+def test_forward_and_gradient_at_partial_tiles(rf, nx, nvec, nu):
+    """Block and node counts that leave part of a 16-block pass, a 4-block step
+    or a 4-node wave, and vector counts that leave part of a workgroup: M against
+    the oracle (FP64 sums of at most 96 terms), the loss against the oracle, and
+    the gradient along a random direction against a central difference of the
+    oracle's loss (truncation d^2 and rounding eps / d of the loss, d = 1e-5)."""
+    p = meshes.tet_block(nx, seed=11)
+    cp, ri, v = lower_of(p)
+    prm = mpnn.init_params(3, out_scale=0.2)
+    h = rf.Mpnn(p.n, cp, ri, v)
+    print(f"case mpnn partial tiles tet{nx} n={p.n} nvec={nvec} nu={nu}", flush=True)
+    optr, oidx, oblk = mpnn.bsr_from_lower(p.n, cp, ri, v)
+    om = mpnn.smoother(prm, optr, oidx, oblk)
+    assert np.max(np.abs(h.smoother(prm)[2] - om)) <= 1e-12 * np.max(np.abs(om))
+    rng = np.random.default_rng(4)
+    e0 = rng.standard_normal((p.n, nvec))
+    loss, g = h.loss(prm, e0, nu=nu, grad=True)
+    assert np.isclose(loss, mpnn.loss(prm, optr, oidx, oblk, e0, nu=nu), rtol=1e-11)
+    d = rng.standard_normal(prm.size) / np.sqrt(prm.size)
+    step = 1e-5
+    fd = (mpnn.loss(prm + step * d, optr, oidx, oblk, e0, nu=nu) -
+          mpnn.loss(prm - step * d, optr, oidx, oblk, e0, nu=nu)) / (2 * step)
+    assert abs(fd - g @ d) <= 1e-6 * np.linalg.norm(g) + 1e-9 * abs(loss)
+
+
 def test_learned_smoother_in_fcg(rf, ora):
     """The network's starting point (zero output layer: scaled damped Jacobi)
     and a random small output layer as finest smoother of AMG-FCG."""
