@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "gemm_kernel.hpp"
+#include "lane_ops.hpp"
 #include "panel_kernels.hpp"
 #include "gpu.hpp"
 
@@ -869,25 +870,6 @@ __global__ __launch_bounds__(64 * NW) void k_sfwd_rows(const FrontDesc* __restri
     if (tid < SRB && valid)
       for (int j = 0; j < nr; ++j) tf[(j0 + j) * tv + r] -= wave_tree_sum<NW>(red, lane, j);
   }
-}
-
-// 32-bit DPP move of both halves of a double (CTRL: a DPP control code)
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-  const long long b = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, 0xF, 0xF, false);
-  return __builtin_bit_cast(double, (static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-
-// sum over the 16 lanes of a DPP row, returned in every lane of the row:
-// quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_ror:4, row_ror:8
-__device__ __forceinline__ double row16_sum(double v) {
-  v += dpp_d<0xB1>(v);
-  v += dpp_d<0x4E>(v);
-  v += dpp_d<0x124>(v);
-  v += dpp_d<0x128>(v);
-  return v;
 }
 
 // partial[tile][j][c] = sum over the tile's rows of L[r, c] t[r][j], c in [c0, c1)

@@ -48,6 +48,50 @@ def test_ic0_apply_matches_oracle(rf, ora, case):
         assert rel_err(z, zo) < 1e-12
 
 
+def first_column(n):
+    """Every row depends on row 0 alone: two levels, n - 1 rows in the second."""
+    a = sp.diags([4.0 + np.arange(n) % 3], [0], format="lil")
+    a[1:, 0] = -1.0 / n
+    a[0, 1:] = -1.0 / n
+    return sp.csc_matrix(a)
+
+
+def random_dense(n):
+    b = np.random.default_rng(n).standard_normal((n, n))
+    return b @ b.T + n * np.eye(n)
+
+
+SWEEPS = {"hex5": lambda: meshes.hex_block(5).to_scipy(),                  # groups of three rows
+          "hex12x3x7": lambda: meshes.hex_block(12, 3, 7).to_scipy(),
+          "plate31x9": lambda: meshes.plate_cpe4(31, 9, 1e11, 0.3, nrhs=1).to_scipy(),  # of two
+          "laplace9": lambda: meshes.laplacian3d(9).to_scipy(),            # of one
+          "one": lambda: np.array([[2.0]]), "diagonal": lambda: np.diag(np.arange(1.0, 130.0)),
+          "dense41": lambda: random_dense(41),    # rows longer than a lane's registers, group of all rows cut
+          "dense100": lambda: random_dense(100),
+          "wide": lambda: first_column(19900),    # the whole ring in use
+          "too_wide": lambda: first_column(20100)}  # a dependency beyond it: launches per level
+
+
+@pytest.mark.parametrize("case", sorted(SWEEPS))
+def test_ic0_sweep_matches_launches_per_level(rf, ora, monkeypatch, case):
+    """The one-workgroup sweeps against one launch per row level and the oracle
+    (the same sums in another order: FP64 rounding of at most 1,000 terms)."""
+    a = SWEEPS[case]()
+    low = lower_csc(a)
+    n = len(low[0]) - 1
+    print(f"case ic0 sweep {case} n={n}", flush=True)
+    s = rf.Pcg(n, *low, kind="ic0")
+    monkeypatch.setenv("RUSTYFEM_IC0_LEVELS", "1")
+    t = rf.Pcg(n, *low, kind="ic0")
+    rng = np.random.default_rng(12)
+    for _ in range(2):
+        r = rng.standard_normal(n)
+        z = s.precondition(r)
+        assert rel_err(z, t.precondition(r)) < 1e-13
+        assert rel_err(z, ora.precond_apply(n, *low, r, kind="ic0")) < 1e-12
+        assert np.array_equal(s.precondition(r), z)
+
+
 def test_ic0_kershaw_shift_matches_oracle(rf, ora):
     a = np.array([[3., -2., 0., 2.], [-2., 3., -2., 0.], [0., -2., 3., -2.], [2., 0., -2., 3.]])
     low = lower_csc(a)
