@@ -31,6 +31,7 @@
 #include <unordered_map>
 
 #include "indef.hpp"
+#include "lane_ops.hpp"
 
 namespace rf {
 
@@ -77,25 +78,16 @@ struct ITile { int32_t rec, r0, c0, pad; };
 struct IEaTile { int32_t crec, prec, x0, y0, nr, cnp; int64_t moff; };
 
 // ---------------------------------------------------------------------------
-// block-wide reductions (256 threads, 4 waves)
+// block-wide reductions (NT threads)
 
+template <int NT = ITH>
 __device__ __forceinline__ double block_max(double v, double* red) {
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   double r = red[0];
-  for (int w = 1; w < NW; ++w) r = fmax(r, red[w]);
-  return r;
-}
-
-__device__ __forceinline__ double block_sum(double v, double* red) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double r = red[0];
-  for (int w = 1; w < NW; ++w) r += red[w];
+  for (int w = 1; w < NT / 64; ++w) r = fmax(r, red[w]);
   return r;
 }
 
@@ -108,6 +100,7 @@ __device__ __forceinline__ void vk_better(double& v, int64_t& k, double ov, int6
   }
 }
 
+template <int NT = ITH>
 __device__ __forceinline__ int64_t block_argmax(double v, int64_t k, double* red, int64_t* redk) {
   for (int o = 32; o > 0; o >>= 1) {
     const double ov = __shfl_xor(v, o, 64);
@@ -122,26 +115,28 @@ __device__ __forceinline__ int64_t block_argmax(double v, int64_t k, double* red
   __syncthreads();
   double bv = red[0];
   int64_t bk = redk[0];
-  for (int w = 1; w < NW; ++w) vk_better(bv, bk, red[w], redk[w]);
+  for (int w = 1; w < NT / 64; ++w) vk_better(bv, bk, red[w], redk[w]);
   return bk;
 }
 
 // max |c[i]| over i in [p, m), i != x1, i != x2 (src/sparse/indef.rs:277-285)
+template <int NT = ITH>
 __device__ double colmax(const double* c, int m, int p, int x1, int x2, double* red) {
   double g = 0.0;
-  for (int i = p + static_cast<int>(threadIdx.x); i < m; i += ITH)
+  for (int i = p + static_cast<int>(threadIdx.x); i < m; i += NT)
     if (i != x1 && i != x2) g = fmax(g, fabs(c[i]));
-  return block_max(g, red);
+  return block_max<NT>(g, red);
 }
 
 // ---------------------------------------------------------------------------
-// LDL^T pivoting steps (one block of 256 threads per front)
+// LDL^T pivoting steps (one workgroup of NT threads per front)
 
 // symmetric interchange of candidate positions p and q (src/sparse/indef.rs:262-273)
+template <int NT = ITH>
 __device__ void iswap(double* G, int m, int kf, int64_t* fs, int p, int q) {
   if (p == q) return;
   const int tid = threadIdx.x;
-  for (int c = tid; c < kf; c += ITH) {
+  for (int c = tid; c < kf; c += NT) {
     double* col = G + static_cast<size_t>(c) * m;
     const double t = col[p];
     col[p] = col[q];
@@ -150,7 +145,7 @@ __device__ void iswap(double* G, int m, int kf, int64_t* fs, int p, int q) {
   __syncthreads();
   double* cp = G + static_cast<size_t>(p) * m;
   double* cq = G + static_cast<size_t>(q) * m;
-  for (int i = tid; i < m; i += ITH) {
+  for (int i = tid; i < m; i += NT) {
     const double t = cp[i];
     cp[i] = cq[i];
     cq[i] = t;
@@ -164,6 +159,7 @@ __device__ void iswap(double* G, int m, int kf, int64_t* fs, int p, int q) {
 }
 
 // 1x1 pivot at p, columns (p, bend) updated for every row (src/sparse/indef.rs:375-389)
+template <int NT = ITH>
 __device__ double ielim1(double* G, int m, int p, int bend, double* wl) {
   const int tid = threadIdx.x;
   double* cp = G + static_cast<size_t>(p) * m;
@@ -172,23 +168,34 @@ __device__ double ielim1(double* G, int m, int p, int bend, double* wl) {
   for (int c0 = 0; c0 < nw; c0 += WCAP) {
     const int cn = min(WCAP, nw - c0);
     __syncthreads();
-    for (int q = tid; q < cn; q += ITH) wl[q] = cp[p + 1 + c0 + q];
+    for (int q = tid; q < cn; q += NT) wl[q] = cp[p + 1 + c0 + q];
     __syncthreads();
-    for (int i = p + 1 + tid; i < m; i += ITH) {
+    for (int i = p + 1 + tid; i < m; i += NT) {
       const double li = cp[i] / dp;
       if (li != 0.0) {
+        // eight columns' loads before their stores: they may not pass a store
+        // to the same array by themselves
         double* row = G + static_cast<size_t>(p + 1 + c0) * m + i;
-        for (int q = 0; q < cn; ++q) row[static_cast<size_t>(q) * m] -= li * wl[q];
+        int q = 0;
+        for (; q + 8 <= cn; q += 8) {
+          double v[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) v[u] = row[static_cast<size_t>(q + u) * m];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) row[static_cast<size_t>(q + u) * m] = v[u] - li * wl[q + u];
+        }
+        for (; q < cn; ++q) row[static_cast<size_t>(q) * m] -= li * wl[q];
       }
     }
   }
   __syncthreads();
-  for (int i = p + 1 + tid; i < m; i += ITH) cp[i] = cp[i] / dp;
+  for (int i = p + 1 + tid; i < m; i += NT) cp[i] = cp[i] / dp;
   __syncthreads();
   return dp;
 }
 
 // 2x2 pivot at (p, p+1) (src/sparse/indef.rs:392-411); returns a, b, c
+template <int NT = ITH>
 __device__ void ielim2(double* G, int m, int p, int bend, double* wl, double& oa, double& ob, double& oc) {
   const int tid = threadIdx.x;
   double* c0p = G + static_cast<size_t>(p) * m;
@@ -200,12 +207,12 @@ __device__ void ielim2(double* G, int m, int p, int bend, double* wl, double& oa
   for (int q0 = 0; q0 < nw; q0 += H) {
     const int cn = min(H, nw - q0);
     __syncthreads();
-    for (int q = tid; q < cn; q += ITH) {
+    for (int q = tid; q < cn; q += NT) {
       wl[q] = c0p[p + 2 + q0 + q];
       wl[H + q] = c1p[p + 2 + q0 + q];
     }
     __syncthreads();
-    for (int i = p + 2 + tid; i < m; i += ITH) {
+    for (int i = p + 2 + tid; i < m; i += NT) {
       const double x0 = c0p[i], x1 = c1p[i];
       const double l0 = (x0 * c - x1 * b) / det;
       const double l1 = (x1 * a - x0 * b) / det;
@@ -216,7 +223,7 @@ __device__ void ielim2(double* G, int m, int p, int bend, double* wl, double& oa
     }
   }
   __syncthreads();
-  for (int i = p + 2 + tid; i < m; i += ITH) {
+  for (int i = p + 2 + tid; i < m; i += NT) {
     const double x0 = c0p[i], x1 = c1p[i];
     c0p[i] = (x0 * c - x1 * b) / det;
     c1p[i] = (x1 * a - x0 * b) / det;
@@ -229,20 +236,21 @@ __device__ void ielim2(double* G, int m, int p, int bend, double* wl, double& oa
 
 // threshold pivot search in [p, end) (src/sparse/indef.rs:287-324):
 // 0 none, 1 one (j), 2 two (j, r)
+template <int NT = ITH>
 __device__ int ichoose(const double* G, int m, int p, int end, const int64_t* fs, const double* scale, double thr,
                        int& oj, int& orr, double* red, int64_t* redk) {
   for (int j = p; j < end; ++j) {
     const double* cj = G + static_cast<size_t>(j) * m;
     const double ajj = cj[j];
     const double sj = scale[fs[j]];
-    const double gj = colmax(cj, m, p, j, -1, red);
+    const double gj = colmax<NT>(cj, m, p, j, -1, red);
     if (fabs(ajj) > ZERO_TOL * sj && fabs(ajj) >= thr * gj) {
       oj = j;
       return 1;
     }
     double best = 0.0;
     int64_t bk = INT64_MAX;
-    for (int i = p + static_cast<int>(threadIdx.x); i < end; i += ITH)
+    for (int i = p + static_cast<int>(threadIdx.x); i < end; i += NT)
       if (i != j) {
         const double v = fabs(cj[i]);
         if (v > best) {
@@ -250,15 +258,15 @@ __device__ int ichoose(const double* G, int m, int p, int end, const int64_t* fs
           bk = i;
         }
       }
-    const int64_t r64 = block_argmax(best, bk, red, redk);
+    const int64_t r64 = block_argmax<NT>(best, bk, red, redk);
     if (r64 == INT64_MAX) continue;
     const int r = static_cast<int>(r64);
     const double a = ajj, b = cj[r], cc = G[static_cast<size_t>(r) * m + r];
     const double det = a * cc - b * b;
     const double sr = scale[fs[r]];
     if (!(fabs(det) > ZERO_TOL * sj * sr)) continue;
-    const double gj2 = colmax(cj, m, p, j, r, red);
-    const double gr2 = colmax(G + static_cast<size_t>(r) * m, m, p, r, j, red);
+    const double gj2 = colmax<NT>(cj, m, p, j, r, red);
+    const double gr2 = colmax<NT>(G + static_cast<size_t>(r) * m, m, p, r, j, red);
     const double ad = fabs(det);
     if ((fabs(cc) * gj2 + fabs(b) * gr2) / ad <= 1.0 / thr && (fabs(b) * gj2 + fabs(a) * gr2) / ad <= 1.0 / thr) {
       oj = j;
@@ -271,11 +279,12 @@ __device__ int ichoose(const double* G, int m, int p, int end, const int64_t* fs
 
 // Bunch-Kaufman choice over the remaining candidates of a root
 // (src/sparse/indef.rs:326-372): returns -1 with kind/j/r, or the singular equation
+template <int NT = ITH>
 __device__ int64_t ichoose_forced(const double* G, int m, int p, int kf, const int64_t* fs, const double* scale,
                                   int& kind, int& oj, int& orr, double* red, int64_t* redk) {
   double big = -1.0;
   int64_t key = INT64_MAX;
-  for (int j = p + static_cast<int>(threadIdx.x); j < kf; j += ITH) {
+  for (int j = p + static_cast<int>(threadIdx.x); j < kf; j += NT) {
     const double* cj = G + static_cast<size_t>(j) * m;
     for (int i = j; i < kf; ++i) {
       const double v = fabs(cj[i]);
@@ -301,7 +310,7 @@ __device__ int64_t ichoose_forced(const double* G, int m, int p, int kf, const i
   __syncthreads();
   double lam = red[0];
   int64_t lk = redk[0];
-  for (int w = 1; w < NW; ++w) vk_better(lam, lk, red[w], redk[w]);
+  for (int w = 1; w < NT / 64; ++w) vk_better(lam, lk, red[w], redk[w]);
   int bj = p, bi = p;
   if (lk != INT64_MAX) {
     bj = static_cast<int>(lk / kf);
@@ -324,12 +333,12 @@ __device__ int64_t ichoose_forced(const double* G, int m, int p, int kf, const i
   const double ajj = fabs(diag(j));
   if (ajj >= ALPHA * lam) return one(j);
   double sig = 0.0;
-  for (int i = p + static_cast<int>(threadIdx.x); i < kf; i += ITH) {
+  for (int i = p + static_cast<int>(threadIdx.x); i < kf; i += NT) {
     if (i == r) continue;
     const double v = fabs(i >= r ? G[static_cast<size_t>(r) * m + i] : G[static_cast<size_t>(i) * m + r]);
     sig = fmax(sig, v);
   }
-  sig = block_max(sig, red);
+  sig = block_max<NT>(sig, red);
   if (ajj * sig >= ALPHA * lam * lam) return one(j);
   if (fabs(diag(r)) >= ALPHA * sig) return one(r);
   const double a = diag(j), b = G[static_cast<size_t>(j) * m + r], cc = diag(r);
@@ -352,11 +361,47 @@ __device__ __forceinline__ void put_piv(const IRec& R, int p, double d, double e
 // progress over the remaining candidates; a root then takes Bunch-Kaufman
 // pivots for the rest.  The trailing update and the symmetric copy of the
 // block run in the two kernels that follow.
-__global__ __launch_bounds__(ITH) void k_ipanel(const IRec* __restrict__ recs, IState* st, int base,
-                                                const double* __restrict__ scale, double thr) {
-  __shared__ double wl[WCAP];
-  __shared__ double red[NW];
-  __shared__ int64_t redk[NW];
+//
+// The common step -- the block's next candidate passes the threshold test
+// where it stands -- runs from registers: a thread owns RPT rows of the front
+// and holds them for CB columns at a time (16; 8 with two rows, which fit the
+// registers of 16 waves).  A column block is first updated by
+// the pivots already taken (one read of L per CB columns), then its pivots
+// follow one another with one barrier each: the owners of the panel's rows
+// leave the candidate's entries there in LDS (its unscaled column is the
+// multipliers' other factor), and after the barrier every thread tests its own
+// rows (|a_pp| >= thr max |a_ip| holds when |a_pp| >= thr |a_ip| for each i: a
+// product with thr rounds monotonically) and updates its registers as if the
+// test passed; a failure anywhere is seen after the next barrier, before the
+// pivot's column is stored.  Each entry receives the same
+// products and subtractions in the same order as in the step-by-step
+// elimination (a pivot's update of a column is only done later), so all values
+// and decisions are identical.  When a candidate fails, the columns are
+// brought up to date and that pivot goes through the full search with
+// interchanges and 2 x 2 pivots (ichoose, iswap, ielim1/2); so does everything
+// in a front with more than NT RPT rows or a widened block.
+//
+// Bound by the instructions its one compute unit issues (16 waves: about 100
+// of them per pivot and wave).  32^3 shifted Laplacian, 41 launches per
+// factorization: 1,087 us per launch when every pivot updated the rest of the
+// panel in memory, 172 (one row per thread) and 265 us (two) with the columns in
+// registers and the maximum reduced across the workgroup per pivot, 102 and 189
+// us now.
+
+template <int NT, int RPT, int CB>
+__global__ __launch_bounds__(NT) void k_ipanel(const IRec* __restrict__ recs, IState* st, int base,
+                                               const double* __restrict__ scale, double thr) {
+  // the full search's buffers and the register path's multipliers are not
+  // live together
+  __shared__ union {
+    double wl[WCAP];
+    double wu[IB + 1][IB];  // wu[q][c]: unscaled entry of the segment's pivot q at panel row c (one row of slack)
+  } sh;
+  __shared__ double red[16];
+  __shared__ int64_t redk[16];
+  __shared__ double ajj_s[2], ssc[IB];
+  __shared__ int32_t bad_s[2];
+  static_assert(CB % 2 == 0, "the buffers alternate across column blocks");
   const IRec R = recs[base + blockIdx.x];
   IState* S = st + base + blockIdx.x;
   const int tid = threadIdx.x;
@@ -371,20 +416,143 @@ __global__ __launch_bounds__(ITH) void k_ipanel(const IRec* __restrict__ recs, I
   int p = S->p, width = S->width;
   const int p0 = p;
   const int b1 = min(p + width, kf);
+  const bool fast = m - p0 <= NT * RPT && b1 - p0 <= IB;
+  // the thread's rows
+  int row[RPT];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) row[r] = p0 + tid + r * NT;
+  if (tid < 2) bad_s[tid] = 0;
+  // pivot q has passed: its column of L (the pivot itself in its own row)
+  auto accept = [&](int q, const double (&l)[RPT]) {
+#pragma unroll
+    for (int r = 0; r < RPT; ++r)
+      if (row[r] >= q && row[r] < m) G[static_cast<size_t>(q) * m + row[r]] = l[r];
+    if (row[0] == q) put_piv(R, q, l[0], 0.0, 1);
+  };
+  // v = the columns [c0, c0 + cw) of the thread's rows from p1 on, with the
+  // segment's pivots [seg, p1) applied (QB pivots' multipliers in flight; those
+  // past p1 are 0; columns past cw hold no values)
+  auto columns = [&](double (&v)[RPT][CB], int seg, int c0, int cw, int p1) {
+#pragma unroll
+    for (int r = 0; r < RPT; ++r)
+#pragma unroll
+      for (int c = 0; c < CB; ++c)
+        v[r][c] = (c < cw && row[r] >= p1 && row[r] < m) ? G[static_cast<size_t>(c0 + c) * m + row[r]] : 0.0;
+    constexpr int QB = RPT == 1 ? 8 : 4;
+    for (int q0 = seg; q0 < p1; q0 += QB) {
+      double l[RPT][QB];
+#pragma unroll
+      for (int r = 0; r < RPT; ++r)
+#pragma unroll
+        for (int u = 0; u < QB; ++u)
+          l[r][u] = (q0 + u < p1 && row[r] >= p1 && row[r] < m) ? G[static_cast<size_t>(q0 + u) * m + row[r]] : 0.0;
+#pragma unroll
+      for (int u = 0; u < QB; ++u) {
+        const double* w = &sh.wu[min(q0 + u, p1 - 1) - seg][c0 - p0];
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+          if (l[r][u] != 0.0) {
+#pragma unroll
+            for (int c = 0; c < CB; ++c) v[r][c] -= l[r][u] * w[c];
+          }
+      }
+    }
+  };
   while (p < b1) {
+    if (fast) {
+      const int seg = p;  // every panel column is up to date with the pivots before seg
+      bool stop = false;
+      if (tid < b1 - seg) ssc[seg - p0 + tid] = scale[R.fs[seg + tid]];
+      int c0 = seg;
+      while (c0 < b1 && !stop) {
+        const int cw = min(CB, b1 - c0);
+        double v[RPT][CB];
+        columns(v, seg, c0, cw, c0);
+        // the block's pivots; the threshold test of pivot p is known complete
+        // after the barrier of pivot p + 1 (or the one after the loop)
+        double lp[RPT];  // column p - 1 of L, stored once its test has passed
+        bool any = false;
+#pragma unroll
+        for (int jj = 0; jj < CB; ++jj) {
+          if (jj >= cw || stop) continue;
+          const int par = jj & 1, np = p - seg;
+          if (row[0] == p) ajj_s[par] = v[0][jj];
+          if (row[0] > p && row[0] < b1) sh.wu[np][row[0] - p0] = v[0][jj];
+          lds_barrier();  // the stores of L are the thread's own until the panel ends
+          if (any) {
+            if (bad_s[par ^ 1]) {
+              stop = true;
+              continue;
+            }
+            accept(p - 1, lp);
+          }
+          const double dp = ajj_s[par];
+          // a pivot that is too small for itself fails for every thread
+          bool bad = !(fabs(dp) > ZERO_TOL * ssc[p - p0]);
+          const double* w = &sh.wu[np][c0 - p0];
+#pragma unroll
+          for (int r = 0; r < RPT; ++r) {
+            if (row[r] > p && row[r] < m) {
+              bad = bad || fabs(v[r][jj]) * thr > fabs(dp);
+              const double li = v[r][jj] / dp;
+              lp[r] = li;
+              if (li != 0.0) {
+#pragma unroll
+                for (int c = jj + 1; c < CB; ++c) v[r][c] -= li * w[c];
+              }
+            } else {
+              lp[r] = dp;
+            }
+          }
+          if (bad) bad_s[par] = 1;
+          any = true;
+          ++p;
+        }
+        lds_barrier();
+        if (stop) {
+          --p;  // the pivot whose test failed
+        } else if (bad_s[(cw - 1) & 1]) {
+          stop = true;
+          --p;
+        } else {
+          accept(p - 1, lp);
+        }
+        if (stop) {
+          // its update went into the registers: the panel's columns from it
+          // on are taken up again from memory
+          c0 = p;
+          lds_barrier();
+          if (tid < 2) bad_s[tid] = 0;
+        } else {
+          c0 += cw;
+        }
+      }
+      for (; c0 < b1; c0 += CB) {
+        const int cw = min(CB, b1 - c0);
+        double v[RPT][CB];
+        columns(v, seg, c0, cw, p);
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+#pragma unroll
+          for (int c = 0; c < CB; ++c)
+            if (c < cw && row[r] >= p && row[r] < m) G[static_cast<size_t>(c0 + c) * m + row[r]] = v[r][c];
+      }
+      __syncthreads();
+      if (p >= b1) break;
+    }
     int j = 0, r = 0;
-    const int kd = ichoose(G, m, p, b1, R.fs, scale, thr, j, r, red, redk);
+    const int kd = ichoose<NT>(G, m, p, b1, R.fs, scale, thr, j, r, red, redk);
     if (kd == 1) {
-      iswap(G, m, kf, R.fs, p, j);
-      const double dp = ielim1(G, m, p, b1, wl);
+      iswap<NT>(G, m, kf, R.fs, p, j);
+      const double dp = ielim1<NT>(G, m, p, b1, sh.wl);
       if (tid == 0) put_piv(R, p, dp, 0.0, 1);
       p += 1;
     } else if (kd == 2) {
       const int rr = (r == p) ? j : r;
-      iswap(G, m, kf, R.fs, p, j);
-      iswap(G, m, kf, R.fs, p + 1, rr);
+      iswap<NT>(G, m, kf, R.fs, p, j);
+      iswap<NT>(G, m, kf, R.fs, p + 1, rr);
       double a, b, c;
-      ielim2(G, m, p, b1, wl, a, b, c);
+      ielim2<NT>(G, m, p, b1, sh.wl, a, b, c);
       if (tid == 0) {
         put_piv(R, p, a, b, 2);
         put_piv(R, p + 1, c, 0.0, 0);
@@ -408,22 +576,22 @@ __global__ __launch_bounds__(ITH) void k_ipanel(const IRec* __restrict__ recs, I
   if (fin && R.root && p < kf) {
     while (p < kf) {
       int kd = 0, j = 0, r = 0;
-      const int64_t e = ichoose_forced(G, m, p, kf, R.fs, scale, kd, j, r, red, redk);
+      const int64_t e = ichoose_forced<NT>(G, m, p, kf, R.fs, scale, kd, j, r, red, redk);
       if (e >= 0) {
         err = e;
         break;
       }
       if (kd == 1) {
-        iswap(G, m, kf, R.fs, p, j);
-        const double dp = ielim1(G, m, p, kf, wl);
+        iswap<NT>(G, m, kf, R.fs, p, j);
+        const double dp = ielim1<NT>(G, m, p, kf, sh.wl);
         if (tid == 0) put_piv(R, p, dp, 0.0, 1);
         p += 1;
       } else {
         const int rr = (r == p) ? j : r;
-        iswap(G, m, kf, R.fs, p, j);
-        iswap(G, m, kf, R.fs, p + 1, rr);
+        iswap<NT>(G, m, kf, R.fs, p, j);
+        iswap<NT>(G, m, kf, R.fs, p + 1, rr);
         double a, b, c;
-        ielim2(G, m, p, kf, wl, a, b, c);
+        ielim2<NT>(G, m, p, kf, sh.wl, a, b, c);
         if (tid == 0) {
           put_piv(R, p, a, b, 2);
           put_piv(R, p + 1, c, 0.0, 0);
@@ -890,6 +1058,42 @@ __global__ __launch_bounds__(256) void k_inertia(const IRec* __restrict__ recs, 
 // leaves its update rows for the parent; the pivots' values go to x after
 // D^-1 (LDL^T).  Backward: gathers x of the update rows and back-substitutes.
 
+//
+// The unit lower triangle is taken 64 pivots at a time: one wave solves the
+// diagonal block with its rows in registers (a lane's row of L loaded at once,
+// the solved entry broadcast by a lane read), then every thread applies the
+// block to the rows below (backward: a wave sums each column over the rows
+// below first).  32^3 shifted Laplacian (pivots up to 1,024 per front): one
+// pivot per barrier, its column read after it, 252 / 287 us per level forward
+// / backward; this 60 / 80 us.
+
+constexpr int SB = 64;  // pivots per solve block
+
+// t[b0:b0+bw) <- L_bb^-1 t with L unit lower, for one wave; kind: 2 marks the
+// first pivot of a 2 x 2 block, whose entry of L below it is not a multiplier
+// (null: none)
+__device__ __forceinline__ void wave_lower_solve(const double* __restrict__ G, int m, int b0, int bw,
+                                                 const int32_t* __restrict__ kind, double* t) {
+  const int lane = threadIdx.x & 63, q = min(lane, bw - 1);
+  double x = t[b0 + q];
+  const int kq = kind ? kind[b0 + q] : 1;
+  for (int h = 0; h < bw; h += 16) {
+    double l[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) l[u] = G[static_cast<size_t>(b0 + min(h + u, bw - 1)) * m + b0 + q];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int i = h + u;
+      if (i < bw) {
+        const double ti = readlane_d(x, i);
+        const int first = __builtin_amdgcn_readlane(kq, i) == 2 ? i + 2 : i + 1;
+        if (lane >= first) x -= l[u] * ti;
+      }
+    }
+  }
+  if (lane < bw) t[b0 + lane] = x;
+}
+
 template <bool LU>
 __global__ __launch_bounds__(ITH) void k_ifwd(const IRec* __restrict__ recs, const IState* __restrict__ st,
                                               int base, const int32_t* __restrict__ smap, double* x) {
@@ -898,6 +1102,7 @@ __global__ __launch_bounds__(ITH) void k_ifwd(const IRec* __restrict__ recs, con
   const int tid = threadIdx.x;
   const int m = R.m, kf = R.kf, np = st[r].npiv;
   double* t = R.t;
+  __shared__ double tb[SB];
   for (int q = tid; q < m; q += ITH) {
     double v = 0.0;
     if (q < kf) {
@@ -917,12 +1122,21 @@ __global__ __launch_bounds__(ITH) void k_ifwd(const IRec* __restrict__ recs, con
     __syncthreads();
   }
   const double* G = R.G;
-  for (int i = 0; i < np; ++i) {
-    const double ti = t[i];
-    const int first = (!LU && R.kind[i] == 2) ? i + 2 : i + 1;
-    if (ti != 0.0) {
-      const double* col = G + static_cast<size_t>(i) * m;
-      for (int q = first + tid; q < m; q += ITH) t[q] -= col[q] * ti;
+  for (int b0 = 0; b0 < np; b0 += SB) {
+    const int bw = min(SB, np - b0);
+    if (tid < 64) wave_lower_solve(G, m, b0, bw, LU ? nullptr : R.kind, t);
+    __syncthreads();
+    if (tid < bw) tb[tid] = t[b0 + tid];
+    // a 2 x 2 pivot whose second row starts the next block
+    const bool cross = !LU && R.kind[b0 + bw - 1] == 2;
+    __syncthreads();
+    for (int q = b0 + bw + tid; q < m; q += ITH) {
+      const double* g = G + static_cast<size_t>(b0) * m + q;
+      const int n = cross && q == b0 + bw ? bw - 1 : bw;
+      double v = t[q];
+#pragma unroll 16
+      for (int i = 0; i < n; ++i) v -= g[static_cast<size_t>(i) * m] * tb[i];
+      t[q] = v;
     }
     __syncthreads();
   }
@@ -962,13 +1176,14 @@ __global__ __launch_bounds__(ITH) void k_ifwd(const IRec* __restrict__ recs, con
 template <bool LU>
 __global__ __launch_bounds__(ITH) void k_ibwd(const IRec* __restrict__ recs, const IState* __restrict__ st,
                                               int base, double* x) {
-  __shared__ double red[NW];
   const int r = base + blockIdx.x;
   const IRec R = recs[r];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = R.m, kf = R.kf, np = st[r].npiv;
   double* t = R.t;
   const double* G = R.G;
+  __shared__ double Lb[LU ? 1 : SB][SB + 1];  // Lb[q][i] = L[b0 + q][b0 + i]
+  __shared__ double tb[SB];
   if (LU && R.root && np < kf) {
     const int rd = kf - np;
     double* t2 = t + m;
@@ -1007,23 +1222,45 @@ __global__ __launch_bounds__(ITH) void k_ibwd(const IRec* __restrict__ recs, con
       __syncthreads();
     }
   } else {
-    // t[i] -= L[np:m, i]^T t[np:m], one wave per column
-    for (int i = wave; i < np; i += NW) {
-      const double* col = G + static_cast<size_t>(i) * m;
-      double s = 0.0;
-      for (int q = np + lane; q < m; q += 64) s += col[q] * t[q];
-      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-      if (lane == 0) t[i] -= s;
-    }
-    __syncthreads();
-    for (int i = np - 1; i >= 0; --i) {
-      const double* col = G + static_cast<size_t>(i) * m;
-      const int skip = R.kind[i] == 2 ? i + 1 : -1;
-      double s = 0.0;
-      for (int q = i + 1 + tid; q < np; q += ITH)
-        if (q != skip) s += col[q] * t[q];
-      s = block_sum(s, red);
-      if (tid == 0) t[i] -= s;
+    for (int b0 = np > 0 ? (np - 1) / SB * SB : -1; b0 >= 0; b0 -= SB) {
+      const int bw = min(SB, np - b0), b1 = b0 + bw;
+      // the diagonal block, and the columns' sums over the rows below, four
+      // columns of a wave at a time
+      for (int idx = tid; idx < SB * SB; idx += ITH) {
+        const int q = idx % SB, i = idx / SB;
+        if (q < bw && i < bw) Lb[LU ? 0 : q][i] = G[static_cast<size_t>(b0 + i) * m + b0 + q];
+      }
+      // the entry of L below the first pivot of a 2 x 2 block is no multiplier
+      const bool cross = R.kind[b1 - 1] == 2;
+      for (int i0 = 4 * wave; i0 < bw; i0 += 4 * NW) {
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int q = b1 + lane; q < m; q += 64) {
+          const double tq = t[q];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int i = min(b0 + i0 + u, b1 - 1);
+            const double l = G[static_cast<size_t>(i) * m + q];
+            s[u] += (cross && i == b1 - 1 && q == b1) ? 0.0 : l * tq;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          for (int o = 32; o > 0; o >>= 1) s[u] += __shfl_xor(s[u], o, 64);
+          if (lane == 0 && i0 + u < bw) tb[i0 + u] = t[b0 + i0 + u] - s[u];
+        }
+      }
+      __syncthreads();
+      if (tid < 64) {
+        double v = tb[min(lane, bw - 1)];
+        const int kq = R.kind[b0 + min(lane, bw - 1)];
+        for (int q = bw - 1; q > 0; --q) {
+          const double tq = readlane_d(v, q);
+          const double l = Lb[LU ? 0 : q][min(lane, bw - 1)];
+          if (lane < q && !(kq == 2 && lane == q - 1)) v -= l * tq;
+        }
+        if (lane < bw) t[b0 + lane] = v;
+      }
       __syncthreads();
     }
   }
@@ -1184,6 +1421,17 @@ class IndefImpl final : public IndefGpu {
         for (int r0 = 0; r0 < H.kf; r0 += TT)
           for (int c0 = 0; c0 <= r0; c0 += TT) mirror.push_back({H.rec, r0, c0, 0});
     }
+  }
+
+  // the panel kernel whose threads own every row of the level's largest front
+  // (two rows each from 1,025 on; beyond 2,048 it takes the full search only)
+  void launch_ipanel(int nlv, int32_t maxm, const IRec* recs, IState* state, int base, double thr) {
+    const double* sc = d_scale_.as<double>();
+    if (maxm <= 128) k_ipanel<128, 1, 16><<<nlv, 128, 0, stream_>>>(recs, state, base, sc, thr);
+    else if (maxm <= 256) k_ipanel<256, 1, 16><<<nlv, 256, 0, stream_>>>(recs, state, base, sc, thr);
+    else if (maxm <= 512) k_ipanel<512, 1, 16><<<nlv, 512, 0, stream_>>>(recs, state, base, sc, thr);
+    else if (maxm <= 1024) k_ipanel<1024, 1, 16><<<nlv, 1024, 0, stream_>>>(recs, state, base, sc, thr);
+    else k_ipanel<1024, 2, 8><<<nlv, 1024, 0, stream_>>>(recs, state, base, sc, thr);
   }
 
   Symbolic sym_;
@@ -1361,8 +1609,11 @@ int64_t IndefImpl::factor(const double* vals) {
     if (!lu_ && !mirror.empty())
       k_imirror<<<static_cast<unsigned>(mirror.size()), 256, 0, stream_>>>(d_mirror.as<ITile>(), d_recs, d_state, 1);
     // rounds of pivot blocks until every front of the level has finished
-    int32_t maxkf = 0;
-    for (int32_t f : lv) maxkf = std::max(maxkf, hf_[f].kf);
+    int32_t maxkf = 0, maxm = 0;
+    for (int32_t f : lv) {
+      maxkf = std::max(maxkf, hf_[f].kf);
+      maxm = std::max(maxm, hf_[f].m);
+    }
     const int64_t cap = 4 * static_cast<int64_t>(maxkf) + 64;
     int64_t rounds = 0;
     std::vector<IState> sh(nlv);
@@ -1375,7 +1626,7 @@ int64_t IndefImpl::factor(const double* vals) {
           if (!trail.empty())
             k_ltrail<<<static_cast<unsigned>(trail.size()), 256, 0, stream_>>>(d_trail.as<ITile>(), d_recs, d_state);
         } else {
-          k_ipanel<<<nlv, ITH, 0, stream_>>>(d_recs, d_state, base, d_scale_.as<double>(), thr);
+          launch_ipanel(nlv, maxm, d_recs, d_state, base, thr);
           if (!trail.empty())
             k_itrail<<<static_cast<unsigned>(trail.size()), 256, 0, stream_>>>(d_trail.as<ITile>(), d_recs, d_state);
           if (!mirror.empty())

@@ -152,6 +152,30 @@ def test_delayed_and_2x2_pivots(rf, ora, g, dscale):
     assert relres(p, x, b) < 1e-9
 
 
+@pytest.mark.parametrize("n,weak", [(1, 0.0), (17, 0.3), (64, 0.3), (65, 0.0), (127, 0.3), (129, 0.02), (257, 0.3),
+                                    (300, 0.0), (513, 0.1), (1030, 0.02)])
+def test_dense_fronts_around_the_panel_sizes(rf, ora, n, weak):
+    """Dense symmetric indefinite matrices at the sizes where the panel kernel
+    changes its workgroup or its rows per thread, `weak` of the diagonal so
+    small that the threshold test fails there: interchanges and 2x2 pivots
+    between stretches of ordinary ones."""
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n))
+    a = a + a.T
+    d = np.where(rng.random(n) < 0.5, 1.0, -1.0) * (n + rng.random(n))
+    d[rng.random(n) < weak] *= 1e-6
+    np.fill_diagonal(a, d)
+    p = dense_problem(a)
+    print(f"case dense indefinite n={n} weak={weak}", flush=True)
+    h, err, ine = rf.Handle.factor_indef(p)
+    assert h is not None, rf.last_error()
+    ho, _, ineo = ora.Handle.factor_indef(p)
+    assert list(ine) == list(ineo)
+    assert_same_factor(h, ho)
+    b = np.cos(np.arange(n) * 0.3)
+    assert relres(p, h.solve(b), b) < 1e-9
+
+
 def test_delays_reach_many_levels(rf, ora):
     """A larger strongly indefinite grid with delays at several levels."""
     p = bipartite_grid(10, 3, 1e-3)
