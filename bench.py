@@ -754,11 +754,9 @@ def main():
     achieved = gemm_flops / (gemm_ms * 1e-3) / 1e12 if gemm_ms > 0 else None
     roof = {"bound": "mfma", "achieved": achieved, "peak": PEAK["fp32_mfma_tflops"], "unit": "TFLOP/s",
             "frac": (achieved / PEAK["fp32_mfma_tflops"]) if achieved else None, "traffic": measured_traffic(),
-            "kernel": "k_gemm<float> / k_gemm_agpr<float> / k_gemm_ilv<float> / k_gemm_k64<float> / k_gemm_q "
-                      "(Schur update, v_mfma_f32_16x16x4f32; kernel autotuned per launch)",
-            "autotuned_agpr_launches": st.get("agpr_launches"),
-            "autotuned_double_width_k_launches": st.get("ilv_launches"),
-            "autotuned_16byte_launches": st.get("q_launches"),
+            "kernel": "k_gemm<float> (Schur update, v_mfma_f32_32x32x2f32; tile shape autotuned per launch)",
+            "autotuned_128x64_launches": st.get("ilv_launches"),
+            "autotuned_128x128_launches": st.get("q_launches"),
             "autotune_ms": st.get("tune_ms"),
             "launches": gemm_n, "avg_launch_ms": gemm_ms / gemm_n if gemm_n else None,
             "algorithmic_flops_per_launch": gemm_flops / gemm_n if gemm_n else None}

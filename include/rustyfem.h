@@ -134,17 +134,17 @@ int64_t rustyfem_eigen(const Handle *h, const int64_t *b_indptr, const int64_t *
  * environment variable RUSTYFEM_KERNEL_TIMING=1 was set at factorization;
  * [13] time (ms) of the GEMM autotuning done before the first factorization
  * (RUSTYFEM_AUTOTUNE=0 turns it off), [14] the GEMM launches it timed and
- * [15] how many of them it moved to the AGPR-accumulator kernel,
+ * [15] always 0 (a kernel of earlier versions),
  * [16..19] the worst relative residual after 0, 1, 2 and 3 refinement
  * corrections of the last solve (-1 where not reached), [20] how many GEMM
- * launches the autotuning moved to the kernels with double-width K tiles,
+ * launches the autotuning moved to 128 x 64 tiles,
  * [21] 1 when the last refinement took back a correction that raised the
  * worst residual (the iterate before it is the result), [22] 1 when the last
  * solve of a mixed-precision handle missed the refinement target and was
  * repeated with an FP64 factorization of the same values (built at the first
  * such solve, kept until the next refactorization), [23] the relative
  * residual that repeat reached (-1 if none ran), [24] how many GEMM launches
- * the autotuning moved to the kernel with 16-byte accesses (FP32 only),
+ * the autotuning moved to 128 x 128 tiles (FP32 only),
  * [25] how many tree levels the triangular solves take through the fused
  * per-front kernels (levels whose fronts all have at most 384 rows and 128
  * pivots; with more than four right-hand sides only those of at most 192

@@ -2,572 +2,241 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mf.hpp"
 #include "mfma.hpp"
 
 namespace rf {
 
-// Workgroup bid of a launch runs on XCD bid % 8 (round-robin dispatch).  The
-// tile of bid is chosen so that every XCD works through a contiguous run of
-// the tile list (tiles of one front column block share their B panel, which
-// then stays in that XCD's L2).  A bijection on [0, nb).
-__device__ __forceinline__ int xcd_tile(int bid, int nb) {
-  const int x = bid & 7, s = bid >> 3, q = nb >> 3, r = nb & 7;
-  return x < r ? x * (q + 1) + s : r * (q + 1) + (x - r) * q + s;
+// 16 bytes of consecutive entries at an entry-aligned address: one access
+// (gfx950 runs in unaligned access mode; the front leading dimension m is
+// arbitrary).
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// The MFMA block of the Schur update: BS x BS outputs, KS k per instruction;
+// lane l supplies the first operand's entry [l % BS][l / BS] and the second's
+// [l / BS][l % BS], and its output register e is column ocol(l, e) of the
+// first operand's index, l % BS of the second's.  FP32 takes the 32 x 32
+// block: per k it needs half the LDS operand reads of the 16 x 16 one.
+template <typename T>
+struct GemmMfma;
+template <>
+struct GemmMfma<float> {
+  static constexpr int BS = 32, KS = 2, E = 4, NACC = 16;
+  using acc_t = v16f;
+  using unaligned_t = f4u;
+  using lds_t = v4f;
+  __device__ static acc_t op(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+  __device__ static int ocol(int lane, int e) { return 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3); }
+};
+template <>
+struct GemmMfma<double> {
+  static constexpr int BS = 16, KS = 4, E = 2, NACC = 4;
+  using acc_t = v4d;
+  using unaligned_t = d2u;
+  using lds_t = v2d;
+  __device__ static acc_t op(double a, double b, acc_t c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+  __device__ static int ocol(int lane, int e) { return (lane >> 4) + 4 * e; }
+};
+
+// Workgroup bid of a launch runs on XCD bid % 8 (round-robin dispatch).  Every
+// group of 512 tiles, what the chip holds at once, is dealt to the XCDs in
+// runs of 64: the list goes through a front in blocks of GT_SUPER x GT_SUPER
+// tiles, so a run shares 16 panels, which stay in that XCD's L2, instead of
+// the 64 and more of tiles taken in turn.  The rest of the list stays in turn,
+// so that its fronts of long K spread over the chip.  A bijection on [0, nb).
+template <int NS>
+__device__ __forceinline__ int gemm_order(int bid, int nb) {
+  constexpr int RUN = GT_SUPER * GT_SUPER * NS;
+  const int g = bid / (8 * RUN);
+  if ((g + 1) * 8 * RUN > nb) return bid;
+  const int x = bid & 7, s = (bid % (8 * RUN)) >> 3;
+  return g * 8 * RUN + x * RUN + s;
 }
 
-// C[r0:r0+128, c0:min(c0+128, cend)) -= (L[r0:, k0:k1] D[k0:k1]) L[c0:, k0:k1]^T
-// on one 128 x 128 tile of a column-major front.
+// C[r0:r0+TM, c0:min(c0+TN, cend)) -= (L[r0:, k0:k1] D[k0:k1]) L[c0:, k0:k1]^T
+// on one TM x TN tile of a column-major front.  The launch covers a list of
+// 128 x 128 tiles with NS = (128 / TM)(128 / TN) workgroups each; one whose
+// part starts outside the tile's valid rows and columns or lies above the
+// diagonal returns at once (NS = 1 with a smaller tile is for lists of tiles
+// that need no more than their first part).
 //
-// Four waves, 2 x 2, each own a 64 x 64 block (4 x 4 MFMA 16 x 16 outputs).
-// The MFMA row index runs over C's columns, so that lanes 0..15 of an output
-// register hold 16 consecutive rows of the front (coalesced C access).
+// Four waves, 2 x 2, each own a TM/2 x TN/2 block.  The MFMA's first operand
+// runs over C's columns, so that the lanes of an output register hold BS
+// consecutive rows of the front (coalesced C access).
+//  - Global loads: 16 bytes down a column of each panel per thread.  A group
+//    of rows that starts at or beyond the last valid row starts at that row
+//    instead; it then reads up to E - 1 entries past the column (the next
+//    column's unused upper part, or the arena's padding), which reach only C
+//    entries that are not stored.  Columns beyond k1 are clamped to k1 - 1 and
+//    their D is 0; no load carries a mask.
+//  - LDS holds KT columns as they lie in the front, [k][row], so a thread's
+//    loads are stored as they are and an MFMA operand read is one entry per
+//    lane along the rows (consecutive banks).  D multiplies the B panel at the
+//    store.  Two buffers, one barrier per KT columns.
+//  - PD tiles of KT columns are in flight in registers, in straight-line code:
+//    each step issues the loads PD tiles ahead, the products of the current
+//    tile, then stores the next tile.
+// An accumulator receives its products in the order of k whatever the tile, so
+// every shape gives identical results.
 //
-// K tiles of KT columns (32 in FP32, 16 in FP64) are staged in LDS with k
-// contiguous per row: a lane's MFMA steps read their A, B and D operands with
-// 16-byte LDS reads (four steps per read in FP32, two in FP64; lane group
-// g = lane / 16 uses k = 16 h + 4 g + s at step s of chunk h, for both
-// operands).  Row
-// pitch KT + 16 bytes keeps the 16-lane reads on distinct banks.
-//
-// Loads carry no per-element masks, so that the next K tile stays in flight
-// behind the current tile's products: rows beyond the front (A) or beyond
-// cend (B) are clamped to the last valid row, whose finite lower-triangle
-// values reach only C entries that are not stored; columns beyond k1 are
-// clamped to k1 - 1 and their D is 0.  Column addresses are wave-uniform.
-// The C tile is read 16 entries at a time before it is written, so that the
-// reads of a group overlap.
-template <typename T>
+// Bound by the MFMA rate where K and the tile count are large, by C traffic
+// and the fill of the chip where K is small.  Measured TFLOP/s of a front of m
+// rows, K pivots, FP32 128 x 128 / 128 x 64 / 64 x 64 (FP64 128 x 64 / 64 x 64):
+//   m = 18000, K = 3000 (7021 tiles): 127 / 122 / 109   (65 / 56)
+//   m = 16383, K =  256 (8001 tiles): 102 / 102 / 102   (55 / 54)
+//   m =  3001, K =  256  (253 tiles):  61 /  62 /  64   (36 / 39)
+//   m =  2500, K = 1000   (78 tiles):  28 /  45 /  47   (24 / 26)
+// against 118, 91, 55 and 21 (64, 52, 32 and 14) of the best of five kernels
+// with 128 x 128 tiles, k-contiguous LDS rows, 16 x 16 blocks and one tile of
+// up to 64 (32) columns in flight; without the list's order by blocks the FP64
+// 128 x 64 shape reached 59 at the first size.
+template <typename T, int TM, int TN, int KT, int PD, int NS>
 __device__ __forceinline__ void gemm_tile(const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles,
                                           T* __restrict__ arena, const double* __restrict__ dpiv) {
-  using M = Mfma<T>;
-  using V4 = typename M::acc_t;
-  using L16 = typename M::lds16_t;
-  constexpr int E = 16 / static_cast<int>(sizeof(T));  // elements per 16-byte LDS read
-  constexpr int KT = M::KT;
-  constexpr int KP = KT + 16 / static_cast<int>(sizeof(T));
-  constexpr int NQ = KT / 8;
-  const GemmTile t = tiles[blockIdx.x];
-  const FrontDesc d = fd[t.front];
-  __shared__ __attribute__((aligned(16))) T As[GT_M][KP];
-  __shared__ __attribute__((aligned(16))) T Bs[GT_M][KP];
-  __shared__ __attribute__((aligned(16))) T Ds[KT];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1, kg = wave >> 1;
-  const int li = tid & 127;
-  T* F = arena + d.off;
-  const int64_t m = d.m;
-  const int arow = min(t.r0 + li, d.m - 1);
-  const int brow = min(t.c0 + li, t.cend - 1);
-  V4 acc[4][4];
-#pragma unroll
-  for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = V4{0, 0, 0, 0};
-  T ra[4 * NQ], rb[4 * NQ];
-  double rd = 0.0;
-  // thread (li, kg) loads row li of both tiles at k = 4 (kg + 2 q) + j
-  auto gload = [&](int kb) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = min(kb + 4 * (kg + 2 * q) + j, t.k1 - 1);
-        const T* col = F + static_cast<int64_t>(c) * m;
-        ra[4 * q + j] = col[arow];
-        rb[4 * q + j] = col[brow];
-      }
-    if (tid < KT) rd = dpiv[d.start + min(kb + tid, t.k1 - 1)];
-  };
-  auto store = [&](int kb) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int k4 = 4 * (kg + 2 * q);
-      lds_put4(&As[li][k4], ra[4 * q], ra[4 * q + 1], ra[4 * q + 2], ra[4 * q + 3]);
-      lds_put4(&Bs[li][k4], rb[4 * q], rb[4 * q + 1], rb[4 * q + 2], rb[4 * q + 3]);
-    }
-    if (tid < KT) Ds[tid] = kb + tid < t.k1 ? static_cast<T>(rd) : T(0);
-  };
-  const int g = lane >> 4, l16 = lane & 15;
-  gload(t.k0);
-  for (int kb = t.k0; kb < t.k1; kb += KT) {
-    __syncthreads();
-    store(kb);
-    __syncthreads();
-    if (kb + KT < t.k1) gload(kb + KT);
-#pragma unroll
-    for (int h = 0; h < KT / 16; ++h)
-#pragma unroll
-      for (int p = 0; p < 4 / E; ++p) {
-        const int kk = 16 * h + 4 * g + E * p;
-        L16 av[4], bv[4];
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi) av[bi] = *reinterpret_cast<const L16*>(&As[wm * 64 + bi * 16 + l16][kk]);
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj) bv[bj] = *reinterpret_cast<const L16*>(&Bs[wn * 64 + bj * 16 + l16][kk]);
-        const L16 dv = *reinterpret_cast<const L16*>(&Ds[kk]);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi) av[bi] *= dv;
-#pragma unroll
-        for (int s = 0; s < E; ++s)
-#pragma unroll
-          for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = M::op(bv[bj][s], av[bi][s], acc[bi][bj]);
-      }
-  }
-#pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
-    const int row = t.r0 + wm * 64 + bi * 16 + l16;
-    const int rowc = min(row, d.m - 1);
-    T cv[4][4];
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int colc = min(t.c0 + wn * 64 + bj * 16 + M::orow(lane, r), t.cend - 1);
-        cv[bj][r] = F[rowc + static_cast<int64_t>(colc) * m];
-      }
-    if (row >= d.m) continue;
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = t.c0 + wn * 64 + bj * 16 + M::orow(lane, r);
-        if (col < t.cend) F[row + static_cast<int64_t>(col) * m] = cv[bj][r] - acc[bi][bj][r];
-      }
-  }
-}
-
-// The 64 x 64 upper-left quarter of gemm_tile's tile, with one wave: for
-// update blocks of at most 64 rows and columns (the small fronts of the lower
-// levels), the other three waves of gemm_tile would only compute entries it
-// does not store.  The wave loads and stages the same K tiles (its lane is
-// the row, all KT columns per lane) and issues the MFMA sequence of
-// gemm_tile's wave 0 (wm = wn = 0), so the results are identical.
-template <typename T>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm64(
-    const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles,
-                                               T* __restrict__ arena, const double* __restrict__ dpiv) {
-  using M = Mfma<T>;
-  using V4 = typename M::acc_t;
-  using L16 = typename M::lds16_t;
-  constexpr int E = 16 / static_cast<int>(sizeof(T));
-  constexpr int KT = M::KT;
-  constexpr int KP = KT + 16 / static_cast<int>(sizeof(T));
-  const GemmTile t = tiles[blockIdx.x];
-  const FrontDesc d = fd[t.front];
-  __shared__ __attribute__((aligned(16))) T As[64][KP];
-  __shared__ __attribute__((aligned(16))) T Bs[64][KP];
-  __shared__ __attribute__((aligned(16))) T Ds[KT];
-  const int lane = threadIdx.x;
-  T* F = arena + d.off;
-  const int64_t m = d.m;
-  const int arow = min(t.r0 + lane, d.m - 1);
-  const int brow = min(t.c0 + lane, t.cend - 1);
-  V4 acc[4][4];
-#pragma unroll
-  for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = V4{0, 0, 0, 0};
-  T ra[KT], rb[KT];
-  double rd = 0.0;
-  auto gload = [&](int kb) {
-#pragma unroll
-    for (int c4 = 0; c4 < KT; ++c4) {
-      const T* col = F + static_cast<int64_t>(min(kb + c4, t.k1 - 1)) * m;
-      ra[c4] = col[arow];
-      rb[c4] = col[brow];
-    }
-    if (lane < KT) rd = dpiv[d.start + min(kb + lane, t.k1 - 1)];
-  };
-  auto store = [&](int kb) {
-#pragma unroll
-    for (int k4 = 0; k4 < KT; k4 += 4) {
-      lds_put4(&As[lane][k4], ra[k4], ra[k4 + 1], ra[k4 + 2], ra[k4 + 3]);
-      lds_put4(&Bs[lane][k4], rb[k4], rb[k4 + 1], rb[k4 + 2], rb[k4 + 3]);
-    }
-    if (lane < KT) Ds[lane] = kb + lane < t.k1 ? static_cast<T>(rd) : T(0);
-  };
-  const int g = lane >> 4, l16 = lane & 15;
-  gload(t.k0);
-  for (int kb = t.k0; kb < t.k1; kb += KT) {
-    __syncthreads();
-    store(kb);
-    __syncthreads();
-    if (kb + KT < t.k1) gload(kb + KT);
-#pragma unroll
-    for (int h = 0; h < KT / 16; ++h)
-#pragma unroll
-      for (int p = 0; p < 4 / E; ++p) {
-        const int kk = 16 * h + 4 * g + E * p;
-        L16 av[4], bv[4];
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi) av[bi] = *reinterpret_cast<const L16*>(&As[bi * 16 + l16][kk]);
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj) bv[bj] = *reinterpret_cast<const L16*>(&Bs[bj * 16 + l16][kk]);
-        const L16 dv = *reinterpret_cast<const L16*>(&Ds[kk]);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi) av[bi] *= dv;
-#pragma unroll
-        for (int s = 0; s < E; ++s)
-#pragma unroll
-          for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = M::op(bv[bj][s], av[bi][s], acc[bi][bj]);
-      }
-  }
-#pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
-    const int row = t.r0 + bi * 16 + l16;
-    const int rowc = min(row, d.m - 1);
-    T cv[4][4];
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int colc = min(t.c0 + bj * 16 + M::orow(lane, r), t.cend - 1);
-        cv[bj][r] = F[rowc + static_cast<int64_t>(colc) * m];
-      }
-    if (row >= d.m) continue;
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = t.c0 + bj * 16 + M::orow(lane, r);
-        if (col < t.cend) F[row + static_cast<int64_t>(col) * m] = cv[bj][r] - acc[bi][bj][r];
-      }
-  }
-}
-
-// gemm_tile with K tiles twice as wide (64 columns in FP32, 32 in FP64: half
-// the barriers per product and twice the time for the next tile's loads to
-// land) and cheaper loads spread among the products.  A column's address is
-// the K tile's first column (one 64-bit base per tile) plus a 32-bit offset,
-// one scalar multiply-add per column instead of a 64-bit product, and the
-// lane's row is a 32-bit vector offset on it.  The next K tile's loads sit in
-// the same basic block as the current tile's MFMAs (the last K tile is peeled
-// off), and a scheduling pattern interleaves them with the first products.
-// Every accumulator receives the same MFMA sequence as in gemm_tile (k in
-// increasing order, four k per 16-byte LDS read in FP32, two in FP64): both
-// give identical results.
-template <typename T, bool PATTERN>
-__device__ __forceinline__ void gemm_tile_ilv(const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles,
-                                              T* __restrict__ arena, const double* __restrict__ dpiv) {
-  using M = Mfma<T>;
-  using V4 = typename M::acc_t;
-  using L16 = typename M::lds16_t;
-  constexpr int E = 16 / static_cast<int>(sizeof(T));
-  constexpr int KT = 2 * M::KT;
-  constexpr int KP = KT + 16 / static_cast<int>(sizeof(T));
-  constexpr int NQ = KT / 8;
-  const GemmTile t = tiles[blockIdx.x];
-  const FrontDesc d = fd[t.front];
-  __shared__ __attribute__((aligned(16))) T As[GT_M][KP];
-  __shared__ __attribute__((aligned(16))) T Bs[GT_M][KP];
-  __shared__ __attribute__((aligned(16))) T Ds[KT];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1, kg = wave >> 1;
-  const int li = tid & 127;
-  T* F = arena + d.off;
-  const int64_t m = d.m;
-  const int arow = min(t.r0 + li, d.m - 1);
-  const int brow = min(t.c0 + li, t.cend - 1);
-  // a front holds m^2 entries, so KT columns of it span far less than 4 GiB
-  const uint32_t mb = static_cast<uint32_t>(m * static_cast<int64_t>(sizeof(T)));
-  const uint32_t aoff = static_cast<uint32_t>(arow) * static_cast<uint32_t>(sizeof(T));
-  const uint32_t boff = static_cast<uint32_t>(brow) * static_cast<uint32_t>(sizeof(T));
-  const char* Fb = reinterpret_cast<const char*>(F);
-  V4 acc[4][4];
-#pragma unroll
-  for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = V4{0, 0, 0, 0};
-  T ra[4 * NQ], rb[4 * NQ];
-  double rd = 0.0;
-  // thread (li, kg) loads row li of both tiles at k = 4 (kg + 2 q) + j; every
-  // thread loads a D entry (the store keeps those of threads < KT)
-  auto gload = [&](int kb) {
-    const char* base = Fb + static_cast<int64_t>(kb) * m * static_cast<int64_t>(sizeof(T));
-    const int lim = t.k1 - 1 - kb;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = min(4 * (kg + 2 * q) + j, lim);
-        const char* col = base + static_cast<uint32_t>(c) * mb;
-        ra[4 * q + j] = *reinterpret_cast<const T*>(col + aoff);
-        rb[4 * q + j] = *reinterpret_cast<const T*>(col + boff);
-      }
-    rd = dpiv[d.start + min(kb + (tid & (KT - 1)), t.k1 - 1)];
-  };
-  auto store = [&](int kb) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int k4 = 4 * (kg + 2 * q);
-      lds_put4(&As[li][k4], ra[4 * q], ra[4 * q + 1], ra[4 * q + 2], ra[4 * q + 3]);
-      lds_put4(&Bs[li][k4], rb[4 * q], rb[4 * q + 1], rb[4 * q + 2], rb[4 * q + 3]);
-    }
-    if (tid < KT) Ds[tid] = kb + tid < t.k1 ? static_cast<T>(rd) : T(0);
-  };
-  const int g = lane >> 4, l16 = lane & 15;
-  auto products = [&]() {
-#pragma unroll
-    for (int h = 0; h < KT / 16; ++h)
-#pragma unroll
-      for (int p = 0; p < 4 / E; ++p) {
-        const int kk = 16 * h + 4 * g + E * p;
-        L16 av[4], bv[4];
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi) av[bi] = *reinterpret_cast<const L16*>(&As[wm * 64 + bi * 16 + l16][kk]);
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj) bv[bj] = *reinterpret_cast<const L16*>(&Bs[wn * 64 + bj * 16 + l16][kk]);
-        const L16 dv = *reinterpret_cast<const L16*>(&Ds[kk]);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi) av[bi] *= dv;
-#pragma unroll
-        for (int s = 0; s < E; ++s)
-#pragma unroll
-          for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = M::op(bv[bj][s], av[bi][s], acc[bi][bj]);
-      }
-  };
-  gload(t.k0);
-  int kb = t.k0;
-  for (; kb + KT < t.k1; kb += KT) {
-    __syncthreads();
-    store(kb);
-    __syncthreads();
-    gload(kb + KT);
-    products();
-    // one load (and the two scalar instructions of its address) after each
-    // of the first 8 NQ products
-    if constexpr (PATTERN) {
-#pragma unroll
-      for (int i = 0; i < 8 * NQ; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x004, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      }
-    }
-  }
-  __syncthreads();
-  store(kb);
-  __syncthreads();
-  products();
-#pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
-    const int row = t.r0 + wm * 64 + bi * 16 + l16;
-    const int rowc = min(row, d.m - 1);
-    T cv[4][4];
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int colc = min(t.c0 + wn * 64 + bj * 16 + M::orow(lane, r), t.cend - 1);
-        cv[bj][r] = F[rowc + static_cast<int64_t>(colc) * m];
-      }
-    if (row >= d.m) continue;
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = t.c0 + wn * 64 + bj * 16 + M::orow(lane, r);
-        if (col < t.cend) F[row + static_cast<int64_t>(col) * m] = cv[bj][r] - acc[bi][bj][r];
-      }
-  }
-}
-
-// Four floats at a 4-byte aligned address: one 16-byte access (gfx950 runs
-// in unaligned access mode; the front leading dimension m is arbitrary).
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-
-// FP32 Schur-update tile with 16-byte accesses: the same 128 x 128 tile and
-// the same MFMA sequence per accumulator as gemm_tile<float> (k = 16 h + 4 g
-// + s at step s of chunk h for lane group g, k increasing), so the results
-// are identical; what differs is the data movement.
-//  - Global loads: thread (rq, kq) loads rows 4 rq .. 4 rq + 3 of the columns
-//    4 kq .. 4 kq + 3 of both panels, four 16-byte loads per panel (a wave
-//    reads two whole 512-byte column segments per load).  A quad of rows
-//    that starts at or beyond the last valid row starts at that row instead;
-//    it then reads up to three entries past the column (the next column's
-//    unused upper part, or the arena's padding), which reach only C rows
-//    that are not stored.  Columns beyond k1 are clamped to k1 - 1 with D = 0.
-//  - LDS: [k quad][row][k % 4], two buffers, one barrier per K tile: the
-//    next tile's loads are in flight during the current tile's products and
-//    land in the other buffer.  D multiplies the A panel when it is stored.
-//    A lane's MFMA operands for four steps are one 16-byte LDS read.
-//  - C: the A panel is the MFMA's first operand, so output register r of
-//    lane l is row 4 (l / 16) + r, column l % 16 of the 16 x 16 block: every
-//    lane reads and writes four consecutive rows of one column (16 bytes);
-//    a quad that crosses the front's last row is stored entry by entry.
-//  - Tile order: xcd_tile.
-__device__ __forceinline__ void gemm_tile_q(const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles,
-                                            float* __restrict__ arena, const double* __restrict__ dpiv) {
-  using M = Mfma<float>;
-  using V4 = M::acc_t;
-  constexpr int KT = M::KT;      // 32 k per tile
-  constexpr int NKQ = KT / 4;    // k quads per tile
-  __shared__ __attribute__((aligned(16))) float S[2][2][NKQ][GT_M][4];  // [buffer][A, B][k quad][row][k % 4]
+  using M = GemmMfma<T>;
+  using U = typename M::unaligned_t;
+  using V = typename M::lds_t;
+  constexpr int WM = TM / 2, WN = TN / 2, BM = WM / M::BS, BN = WN / M::BS, E = M::E;
+  constexpr int QA = TM / E, QB = TN / E;        // 16-byte groups per column
+  constexpr int CA = 256 / QA, CB = 256 / QB;    // columns per load of the workgroup
+  constexpr int LA = KT / CA, LB = KT / CB;      // loads per thread and tile of KT columns
+  static_assert(LA * CA == KT && LB * CB == KT && PD % 2 == 0, "KT columns are whole loads, PD keeps buffer parity");
+  __shared__ __attribute__((aligned(16))) T As[2][KT][TM];
+  __shared__ __attribute__((aligned(16))) T Bs[2][KT][TN];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
-  const int rq = tid & 31, kq = tid >> 5;
-  const int g = lane >> 4, l16 = lane & 15;
-  const GemmTile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
+  const int wg = gemm_order<NS>(blockIdx.x, gridDim.x);
+  const GemmTile t = tiles[wg / NS];
+  const int part = wg % NS;
+  constexpr int NR = NS == 1 ? 1 : GT_M / TM;
+  const int r0 = t.r0 + (part % NR) * TM, c0 = t.c0 + (part / NR) * TN;
   const FrontDesc d = fd[t.front];
-  float* F = arena + d.off;
+  if (r0 >= d.m || c0 >= t.cend || c0 > r0 + TM - 1) return;
+  T* F = arena + d.off;
   const int64_t m = d.m;
-  const int arow = min(t.r0 + 4 * rq, d.m - 1);
-  const int brow = min(t.c0 + 4 * rq, t.cend - 1);
-  // the K tile in flight: its 16-byte row quads of both panels and the D of
-  // its columns (loaded unconditionally, D of the clamped column, so that no
-  // branch waits for the loads before the products)
-  f4u ra[4], rb[4];
-  double rd[4];
-  int kload = 0;
-  auto gload = [&](int kb) {
-    kload = kb;
+  const int qa = tid % QA, ca = tid / QA, qb = tid % QB, cb = tid / QB;
+  const T* pa = F + min(r0 + E * qa, d.m - 1);
+  const T* pb = F + min(c0 + E * qb, t.cend - 1);
+  struct Stage {
+    U ra[LA], rb[LB];
+    double rd[LB];
+    int kl;
+  };
+  auto gload = [&](Stage& s, int kb) {
+    s.kl = kb;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = min(kb + 4 * kq + j, t.k1 - 1);
-      const float* col = F + static_cast<int64_t>(c) * m;
-      ra[j] = *reinterpret_cast<const f4u*>(col + arow);
-      rb[j] = *reinterpret_cast<const f4u*>(col + brow);
-      rd[j] = dpiv[d.start + c];
+    for (int i = 0; i < LA; ++i)
+      s.ra[i] = *reinterpret_cast<const U*>(pa + static_cast<int64_t>(min(kb + ca + CA * i, t.k1 - 1)) * m);
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+      const int c = min(kb + cb + CB * i, t.k1 - 1);
+      s.rb[i] = *reinterpret_cast<const U*>(pb + static_cast<int64_t>(c) * m);
+      s.rd[i] = dpiv[d.start + c];
     }
   };
-  // A thread writes its four rows in a rotated order, row 4 rq + (rr + o) % 4
-  // at write rr, so that the 16-byte writes of 8 (and of 16) consecutive
-  // lanes land on distinct banks (rows 4 rq + rr alone repeat every 4 lanes)
-  const int rot = ((rq >> 1) + (rq >> 3)) & 3;
-  auto pick = [](const f4u& v, int i) { return i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3]; };
-  auto store = [&](int buf) {
-    float dk[4];
+  auto store = [&](const Stage& s, int buf) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dk[j] = kload + 4 * kq + j < t.k1 ? static_cast<float>(rd[j]) : 0.0f;
+    for (int i = 0; i < LA; ++i) {
+      V v;
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int e = (rr + rot) & 3;
-      *reinterpret_cast<v4f*>(&S[buf][0][kq][4 * rq + e][0]) =
-          v4f{pick(ra[0], e) * dk[0], pick(ra[1], e) * dk[1], pick(ra[2], e) * dk[2], pick(ra[3], e) * dk[3]};
-      *reinterpret_cast<v4f*>(&S[buf][1][kq][4 * rq + e][0]) =
-          v4f{pick(rb[0], e), pick(rb[1], e), pick(rb[2], e), pick(rb[3], e)};
+      for (int e = 0; e < E; ++e) v[e] = s.ra[i][e];
+      *reinterpret_cast<V*>(&As[buf][ca + CA * i][E * qa]) = v;
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+      const T dk = s.kl + cb + CB * i < t.k1 ? static_cast<T>(s.rd[i]) : T(0);
+      V v;
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = s.rb[i][e] * dk;
+      *reinterpret_cast<V*>(&Bs[buf][cb + CB * i][E * qb]) = v;
     }
   };
-  V4 acc[4][4];
+  typename M::acc_t acc[BN][BM];
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi)
+  for (int j = 0; j < BN; ++j)
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = V4{0, 0, 0, 0};
+    for (int i = 0; i < BM; ++i)
+#pragma unroll
+      for (int e = 0; e < M::NACC; ++e) acc[j][i][e] = 0;
+  const int lr = lane & (M::BS - 1), lk = lane / M::BS;
   auto products = [&](int buf) {
+    const T* ap = &As[buf][lk][wm * WM + lr];
+    const T* bp = &Bs[buf][lk][wn * WN + lr];
 #pragma unroll
-    for (int h = 0; h < KT / 16; ++h) {
-      const int q = 4 * h + g;
-      v4f av[4], bv[4];
+    for (int k = 0; k < KT; k += M::KS) {
+      T a[BM], b[BN];
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi) av[bi] = *reinterpret_cast<const v4f*>(&S[buf][0][q][wm * 64 + bi * 16 + l16][0]);
+      for (int i = 0; i < BM; ++i) a[i] = ap[k * TM + M::BS * i];
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj) bv[bj] = *reinterpret_cast<const v4f*>(&S[buf][1][q][wn * 64 + bj * 16 + l16][0]);
+      for (int j = 0; j < BN; ++j) b[j] = bp[k * TN + M::BS * j];
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int i = 0; i < BM; ++i)
 #pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-          for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = M::op(av[bi][s], bv[bj][s], acc[bi][bj]);
+        for (int j = 0; j < BN; ++j) acc[j][i] = M::op(b[j], a[i], acc[j][i]);
     }
   };
-  // the C tile's entries of this lane, read before the last K tile's
-  // products so that their latency hides behind them
-  f4u cv[4][4];
-  auto cload = [&]() {
+  const int nt = (t.k1 - t.k0 + KT - 1) / KT;
+  Stage s[PD];
 #pragma unroll
-    for (int bi = 0; bi < 4; ++bi) {
-      const int rowc = min(t.r0 + wm * 64 + bi * 16 + 4 * g, d.m - 1);
-#pragma unroll
-      for (int bj = 0; bj < 4; ++bj) {
-        const int colc = min(t.c0 + wn * 64 + bj * 16 + l16, t.cend - 1);
-        cv[bi][bj] = *reinterpret_cast<const f4u*>(F + rowc + static_cast<int64_t>(colc) * m);
-      }
-    }
-  };
-  gload(t.k0);
-  store(0);
+  for (int p = 0; p < PD; ++p) gload(s[p], t.k0 + p * KT);
+  store(s[0], 0);
   __syncthreads();
-  // every K tile but the last, then the last with the C reads in flight
-  int buf = 0;
-  for (int kb = t.k0; kb + KT < t.k1; kb += KT) {
-    gload(kb + KT);
-    products(buf);
-    store(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-  cload();
-  __builtin_amdgcn_sched_barrier(0);
-  products(buf);
+  int q = 0;
+  for (; q + PD < nt; q += PD) {
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
-    const int row = t.r0 + wm * 64 + bi * 16 + 4 * g;
+    for (int u = 0; u < PD; ++u) {
+      gload(s[u], t.k0 + (q + u + PD) * KT);
+      products(u & 1);
+      store(s[(u + 1) % PD], (u + 1) & 1);
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < PD; ++u) {
+    products(u & 1);
+    if (q + u + 1 >= nt) break;
+    if (u + 1 < PD) store(s[(u + 1) % PD], (u + 1) & 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < BM; ++i) {
+    const int row = r0 + wm * WM + M::BS * i + lr;
+    const int rowc = min(row, d.m - 1);
+    // all reads of a block row before its writes, so that they overlap
+    T cv[BN][M::NACC];
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+#pragma unroll
+      for (int e = 0; e < M::NACC; ++e)
+        cv[j][e] = F[rowc + static_cast<int64_t>(min(c0 + wn * WN + M::BS * j + M::ocol(lane, e), t.cend - 1)) * m];
     if (row >= d.m) continue;
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) {
-      const int col = t.c0 + wn * 64 + bj * 16 + l16;
-      if (col >= t.cend) continue;
-      const f4u o = cv[bi][bj] - f4u{acc[bi][bj][0], acc[bi][bj][1], acc[bi][bj][2], acc[bi][bj][3]};
-      float* p = F + row + static_cast<int64_t>(col) * m;
-      if (row + 3 < d.m) {
-        *reinterpret_cast<f4u*>(p) = o;
-      } else {
+    for (int j = 0; j < BN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (row + r < d.m) p[r] = o[r];
+      for (int e = 0; e < M::NACC; ++e) {
+        const int c = c0 + wn * WN + M::BS * j + M::ocol(lane, e);
+        if (c < t.cend) F[row + static_cast<int64_t>(c) * m] = cv[j][e] - acc[j][i][e];
       }
-    }
   }
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_q(
-    const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles, float* __restrict__ arena,
-    const double* __restrict__ dpiv) {
-  gemm_tile_q(fd, tiles, arena, dpiv);
-}
-
-// The same tile under two register budgets: k_gemm asks for two waves per
-// SIMD (accumulators in VGPRs; FP32 reaches three), k_gemm_agpr leaves the
-// accumulators in AGPRs (two waves per SIMD in FP32, one in FP64).  Which is
-// faster depends on the launch (tile count, K, front sizes); the solver times
-// both on each launch of its plan once and keeps the faster.
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm(
+template <typename T, int TM, int TN, int KT, int PD, int NS, int W>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k_gemm(
     const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles, T* __restrict__ arena,
     const double* __restrict__ dpiv) {
-  gemm_tile<T>(fd, tiles, arena, dpiv);
+  gemm_tile<T, TM, TN, KT, PD, NS>(fd, tiles, arena, dpiv);
 }
 
+enum GemmShape { GEMM_64x64 = 0, GEMM_128x64 = 1, GEMM_128x128 = 2 };
+// FP64 128 x 128 needs 64 accumulator registers more, spills, and is slower
+// than 128 x 64 at every size measured (m = 16383, K = 2048: 61 against 62
+// TFLOP/s, m = 12000, K = 256: 46 against 53): FP64 factors have two shapes.
 template <typename T>
-__global__ __launch_bounds__(256) void k_gemm_agpr(const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles,
-                                                   T* __restrict__ arena, const double* __restrict__ dpiv) {
-  gemm_tile<T>(fd, tiles, arena, dpiv);
-}
-
-// gemm_tile_ilv, two waves per SIMD, with the load interleaving pattern
-// (k_gemm_ilv) and without it, the loads where the compiler puts them
-// (k_gemm_k64)
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_ilv(const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles,
-                                                  T* __restrict__ arena, const double* __restrict__ dpiv) {
-  gemm_tile_ilv<T, true>(fd, tiles, arena, dpiv);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_k64(
-    const FrontDesc* __restrict__ fd, const GemmTile* __restrict__ tiles, T* __restrict__ arena,
-    const double* __restrict__ dpiv) {
-  gemm_tile_ilv<T, false>(fd, tiles, arena, dpiv);
-}
+constexpr int kGemmShapes = std::is_same<T, float>::value ? 3 : 2;
 
 }  // namespace rf

@@ -27,6 +27,7 @@ constexpr int TRS = 64;       // rows per TRSM tile
 constexpr int SR = 1024;      // rows per solve tile (4 per thread)
 constexpr int BC = 256;       // columns per backward tile (one per thread)
 constexpr int GT_M = 128;     // GEMM tile rows
+constexpr int GT_SUPER = 8;   // GEMM tiles are listed in blocks of GT_SUPER x GT_SUPER
 constexpr int ZC = 64;        // columns per arena-clearing tile
 constexpr int EA_T = 64;      // extend-add tile edge (square tiles)
 constexpr int EA_TX = 256;    // rows of a tall extend-add tile (EA_T * EA_T / EA_TX columns)

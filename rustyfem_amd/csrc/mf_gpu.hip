@@ -1716,6 +1716,19 @@ __global__ __launch_bounds__(256) void k_fwd_finish_ys(const FrontDesc* __restri
 // factorization can be captured into a graph)
 __global__ void k_err_reset(unsigned long long* err) { *err = ULLONG_MAX; }
 
+// arbitrary front entries in (-1, 1) and pivots that keep their updates below
+// them, for the launches of the GEMM autotuning
+template <typename T>
+__global__ __launch_bounds__(256) void k_tune_fill(T* __restrict__ a, int64_t na, double* __restrict__ d, int64_t nd) {
+  const int64_t step = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (int64_t i = i0; i < na; i += step) {
+    const uint32_t h = static_cast<uint32_t>(i) * 2654435761u;
+    a[i] = static_cast<T>(static_cast<int32_t>((h ^ (h >> 15)) * 2246822519u)) * static_cast<T>(0x1p-31);
+  }
+  for (int64_t i = i0; i < nd; i += step) d[i] = 0x1p-20;
+}
+
 __global__ void k_gather(const int64_t* __restrict__ map, const double* __restrict__ src, double* __restrict__ dst,
                          int64_t cnt) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -2005,25 +2018,25 @@ class Impl final : public GpuFactor {
       // RUSTYFEM_TUNE_MARGIN: a variant must be this fraction faster to be picked
       const char* tm = std::getenv("RUSTYFEM_TUNE_MARGIN");
       if (tm && *tm) tune_margin_ = 1.0f - static_cast<float>(std::atof(tm));
-      // RUSTYFEM_AUTOTUNE: unset or 1 = time every GEMM kernel per launch,
-      // 0 = k_gemm everywhere, "agpr" = k_gemm_agpr everywhere, "ilv" =
-      // k_gemm_ilv everywhere, "k64" = k_gemm_k64 everywhere, "q" = k_gemm_q
-      // everywhere (FP32; FP64 factors take k_gemm)
+      // RUSTYFEM_AUTOTUNE: unset or 1 = time every GEMM tile shape per launch,
+      // 0 = 64 x 64 tiles everywhere, "128x64" and "128x128" = those
+      // everywhere (FP64 has no 128 x 128: 128 x 64).  The names of earlier
+      // kernels still force one shape: "agpr" and "k64" 64 x 64, "ilv"
+      // 128 x 64, "q" 128 x 128.
       const char* a = std::getenv("RUSTYFEM_AUTOTUNE");
-      const int8_t force = a && std::strcmp(a, "agpr") == 0  ? 1
-                           : a && std::strcmp(a, "ilv") == 0 ? 2
-                           : a && std::strcmp(a, "k64") == 0 ? 3
-                           : a && std::strcmp(a, "q") == 0   ? (kGemmVariants > 4 ? 4 : 0)
-                                                             : 0;
-      autotune_ = !(a && *a == '0') && force == 0;
+      auto is = [a](const char* n) { return a && std::strcmp(a, n) == 0; };
+      const int8_t force = is("128x64") || is("ilv") ? GEMM_128x64
+                           : is("128x128") || is("q") ? std::min<int>(GEMM_128x128, kGemmShapes<T> - 1)
+                                                      : GEMM_64x64;
+      autotune_ = !(a && *a == '0') && force == GEMM_64x64 && !is("64x64") && !is("agpr") && !is("k64");
       gemm_pick_.assign(P_.gemm.size(), force);
       // In a GEMM launch where most tiles update at most 64 rows and columns
-      // (small fronts), those tiles go first in its range and take the
-      // one-wave 64 x 64 kernel, the others the 128 x 128 kernels; in the
-      // other launches a few such tiles (the corners of large fronts, with
-      // long K) stay with the rest, beside which they run
-      // (RUSTYFEM_NO_GEMM64=1: every tile on the 128 x 128 kernels).  A
-      // tile's result does not depend on its place in the launch.
+      // (small fronts), those tiles go first in its range and run as one
+      // 64 x 64 workgroup each, the others in the launch's shape; in the other
+      // launches a few such tiles (the corners of large fronts, with long K)
+      // stay with the rest, beside which they run (RUSTYFEM_NO_GEMM64=1:
+      // every tile in the launch's shape).  A tile's result does not depend on
+      // its place in the launch.
       const char* g64 = std::getenv("RUSTYFEM_NO_GEMM64");
       gemm64_.assign(P_.gemm.size(), 0);
       if (!(g64 && *g64 && *g64 != '0')) {
@@ -2103,7 +2116,7 @@ class Impl final : public GpuFactor {
           slot_maxu_[sl][L] = std::max<int64_t>(slot_maxu_[sl][L], P_.fd[P_.child_slot_fronts[sl][q]].u);
       }
     }
-    // 64 entries of padding: k_gemm_q's 16-byte loads of a quad of rows that
+    // 64 entries of padding: k_gemm's 16-byte loads of a group of rows that
     // starts at a front's last row read up to three entries past its last column
     d_arena_ = dalloc<T>(static_cast<size_t>(P_.arena_elems) + 64, bytes_);
     d_dpiv_ = dalloc<double>(n_, bytes_);
@@ -2514,7 +2527,7 @@ class Impl final : public GpuFactor {
     if (ph.kind != PhaseKind::Gemm128 && ph.kind != PhaseKind::GemmRest)
       throw std::runtime_error("GEMM phase with 64-column tiles is not supported");
     const int64_t n64 = gemm64_[r.begin];
-    if (n64 > 0) launch_on(st, k_gemm64<T>, n64, 64, d_fd_, d_gemm_ + r.begin, d_arena_, d_dpiv_);
+    if (n64 > 0) launch_shape<64, 64, 1>(Range{r.begin, n64}, st);
     if (n64 < r.count) launch_gemm(gemm_pick_[r.begin], Range{r.begin + n64, r.count - n64}, st);
     tm_.gemm_flops += flops;
     if (ktime_) {
@@ -2523,47 +2536,54 @@ class Impl final : public GpuFactor {
     }
   }
 
-  // variant 0 = k_gemm, 1 = k_gemm_agpr, 2 = k_gemm_ilv, 3 = k_gemm_k64,
-  // 4 = k_gemm_q (FP32 only)
-  static constexpr int kGemmVariants = std::is_same<T, float>::value ? 5 : 4;
-  void launch_gemm(int variant, const Range& r, hipStream_t st) {
-    if constexpr (std::is_same<T, float>::value) {
-      if (variant == 4) {
-        launch_on(st, k_gemm_q, r.count, 256, d_fd_, d_gemm_ + r.begin, d_arena_, d_dpiv_);
+  // KT: every thread loads 16 bytes of each panel at least once; W, the waves
+  // per SIMD the registers are cut for, is what the accumulators and the two
+  // tiles in flight leave without spills
+  template <int TM, int TN, int NS>
+  void launch_shape(const Range& r, hipStream_t st) {
+    constexpr bool F32 = std::is_same<T, float>::value;
+    constexpr int KT = F32 && TN == 64 ? 16 : 8;
+    constexpr int W = TM == 64 ? 4 : F32 ? 2 : 3;
+    launch_on(st, k_gemm<T, TM, TN, KT, 2, NS, W>, r.count * NS, 256, d_fd_, d_gemm_ + r.begin, d_arena_, d_dpiv_);
+  }
+  void launch_gemm(int shape, const Range& r, hipStream_t st) {
+    if constexpr (kGemmShapes<T> > 2) {
+      if (shape == GEMM_128x128) {
+        launch_shape<128, 128, 1>(r, st);
         return;
       }
     }
-    if (variant == 1)
-      launch_on(st, k_gemm_agpr<T>, r.count, 256, d_fd_, d_gemm_ + r.begin, d_arena_, d_dpiv_);
-    else if (variant == 2)
-      launch_on(st, k_gemm_ilv<T>, r.count, 256, d_fd_, d_gemm_ + r.begin, d_arena_, d_dpiv_);
-    else if (variant == 3)
-      launch_on(st, k_gemm_k64<T>, r.count, 256, d_fd_, d_gemm_ + r.begin, d_arena_, d_dpiv_);
+    if (shape == GEMM_128x64)
+      launch_shape<128, 64, 2>(r, st);
     else
-      launch_on(st, k_gemm<T>, r.count, 256, d_fd_, d_gemm_ + r.begin, d_arena_, d_dpiv_);
+      launch_shape<64, 64, 4>(r, st);
   }
 
-  // Autotuning of the GEMM kernel: every GEMM launch of the plan runs the
-  // four variants (one warm-up, then three timed launches each, the minimum
-  // kept); a variant replaces the current choice (k_gemm first) only where it
-  // is at least 1% faster (RUSTYFEM_TUNE_MARGIN).  All four give identical
-  // results.  The launches
-  // work on the arena before the first factorization assembles anything in
-  // it; the factorization clears the arena and every level assembles its
-  // fronts before its own GEMMs, so
-  // what they leave there is never read.
+  // Autotuning of the GEMM tile shape: every GEMM launch of the plan runs its
+  // shapes (one warm-up, then three timed launches each, the minimum kept); a
+  // shape replaces the current choice (64 x 64 first: the best for most
+  // launches, the larger ones pay from some thousand tiles or long K on) only
+  // where it is at least 1% faster (RUSTYFEM_TUNE_MARGIN).  All give identical
+  // results.  The launches work on the arena before the first factorization
+  // assembles anything in it, on arbitrary values in (-1, 1) and pivots small
+  // enough to keep them there: on the zeros of fresh memory the chip draws
+  // less power and clocks higher, which favoured the smaller shapes (64^3
+  // block, mixed: 193.2 ms per refactor and solve against 190.8 with 128 x 128
+  // everywhere).  The factorization clears the arena and every level assembles
+  // its fronts before its own GEMMs, so what they leave there is never read.
   void tune_gemm() {
     std::vector<const Phase*> ph;
     for (const LevelPlan& lp : P_.levels)
       for (const Phase& p : lp.phases)
         if ((p.kind == PhaseKind::Gemm128 || p.kind == PhaseKind::GemmRest) && p.r.count > gemm64_[p.r.begin])
           ph.push_back(&p);
-    constexpr int NV = kGemmVariants;
+    constexpr int NV = kGemmShapes<T>;
     std::vector<hipEvent_t> ev(ph.size() * 4 * NV);
     for (auto& e : ev) HIPCHK(hipEventCreate(&e));
     HIPCHK(hipEventRecord(e0_, s_));
+    launch(k_tune_fill<T>, 2048, 256, d_arena_, P_.arena_elems, d_dpiv_, n_);
     for (size_t i = 0; i < ph.size(); ++i) {
-      // the launch's tiles for the 128 x 128 kernels
+      // the launch's tiles beside those of one 64 x 64 workgroup
       const int64_t n64 = gemm64_[ph[i]->r.begin];
       const Range r{ph[i]->r.begin + n64, ph[i]->r.count - n64};
       for (int v = 0; v < NV; ++v) {
@@ -2598,9 +2618,9 @@ class Impl final : public GpuFactor {
     HIPCHK(hipEventElapsedTime(&ms, e0_, e1_));
     tm_.tune_ms = ms;
     tm_.tuned_launches = static_cast<double>(ph.size());
-    tm_.agpr_launches = static_cast<double>(count[1]);
-    tm_.ilv_launches = static_cast<double>(count[2] + count[3]);
-    tm_.q_launches = NV > 4 ? static_cast<double>(count[NV - 1]) : 0.0;
+    tm_.agpr_launches = 0.0;
+    tm_.ilv_launches = static_cast<double>(count[GEMM_128x64]);
+    tm_.q_launches = NV > GEMM_128x128 ? static_cast<double>(count[NV - 1]) : 0.0;
     tuned_ = true;
   }
 
@@ -3050,8 +3070,8 @@ class Impl final : public GpuFactor {
   int nseg_ = 0, segsq_cap_ = 0;
   bool legacy_panel_ = false;
   bool autotune_ = true, tuned_ = false;
-  std::vector<int8_t> gemm_pick_;  // per GEMM launch (by its first tile): the launch_gemm variant
-  std::vector<int32_t> gemm64_;    // per GEMM launch (by its first tile): its leading tiles for the 64 x 64 kernel
+  std::vector<int8_t> gemm_pick_;  // per GEMM launch (by its first tile): its GemmShape
+  std::vector<int32_t> gemm64_;    // per GEMM launch (by its first tile): its leading tiles of one 64 x 64 workgroup
   bool chain_solve_ = false;
   std::vector<int64_t> lvl_maxm_, lvl_maxk_, slot_maxu_[2];
   SmallFront* d_small_ = nullptr;

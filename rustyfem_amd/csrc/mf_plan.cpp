@@ -10,6 +10,19 @@ namespace rf {
 namespace {
 Range take(int64_t begin, int64_t end) { return Range{begin, end - begin}; }
 
+// the lower 128 x 128 tiles of columns [cb, ce) (clipped at cend) and rows
+// [rb, m) of front f, updated with K = [k0, k1), in blocks of GT_SUPER x
+// GT_SUPER (neighbours in the list share their panels)
+void gemm_tiles(std::vector<GemmTile>& out, int32_t f, int32_t rb, int32_t m, int32_t cb, int32_t ce, int32_t cend,
+                int32_t k0, int32_t k1) {
+  constexpr int32_t S = GT_SUPER * GT_M;
+  for (int32_t cs = cb; cs < ce; cs += S)
+    for (int32_t rs = rb; rs < m; rs += S)
+      for (int32_t c0 = cs; c0 < std::min(cs + S, ce); c0 += GT_M)
+        for (int32_t r0 = rs; r0 < std::min(rs + S, m); r0 += GT_M)
+          if (c0 <= r0 + GT_M - 1) out.push_back({f, r0, c0, cend, k0, k1});
+}
+
 int32_t local_index(const Front& p, int64_t eq) {
   if (eq >= p.start && eq < p.start + p.k) return static_cast<int32_t>(eq - p.start);
   auto it = std::lower_bound(p.rows.begin(), p.rows.end(), eq);
@@ -197,9 +210,7 @@ Plan build_plan(const Symbolic& sym, const std::vector<int64_t>& colptr, const s
           const FrontDesc& d = P.fd[f];
           if (d.k <= J1) continue;
           const int32_t cb = part == 0 ? J1 : std::min(J1 + NBO, d.k), ce = part == 0 ? std::min(J1 + NBO, d.k) : d.k;
-          for (int32_t c0 = cb; c0 < ce; c0 += 128)
-            for (int32_t r0 = J1; r0 < d.m; r0 += GT_M)
-              if (c0 <= r0 + GT_M - 1) P.gemm.push_back({f, r0, c0, d.k, J0, J1});
+          gemm_tiles(P.gemm, f, J1, d.m, cb, ce, d.k, J0, J1);
           fl += colflops(cb, ce, d.m);
         }
         phase(part == 0 ? PhaseKind::Gemm128 : PhaseKind::GemmRest, b, static_cast<int64_t>(P.gemm.size()), fl);
@@ -301,9 +312,7 @@ Plan build_plan(const Symbolic& sym, const std::vector<int64_t>& colptr, const s
       const FrontDesc& d = P.fd[f];
       if (d.u == 0 || d.k == 0) continue;
       fl += static_cast<double>(d.u) * (d.u + 1.0) * d.k;
-      for (int32_t c0 = d.k; c0 < d.m; c0 += 128)
-        for (int32_t r0 = d.k; r0 < d.m; r0 += GT_M)
-          if (c0 <= r0 + GT_M - 1) P.gemm.push_back({f, r0, c0, d.m, 0, d.k});
+      gemm_tiles(P.gemm, f, d.k, d.m, d.k, d.m, d.m, 0, d.k);
     }
     phase(PhaseKind::Gemm128, b, static_cast<int64_t>(P.gemm.size()), fl);
   }

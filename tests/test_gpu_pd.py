@@ -327,6 +327,35 @@ def test_gemm_register_layouts_agree(rf, monkeypatch, precision):
     assert h_v.stats()["tuned_launches"] == 0 and h_i.stats()["tuned_launches"] == 0
 
 
+@pytest.mark.parametrize("k,u", [(3, 1), (7, 65), (17, 129), (63, 64), (65, 127), (130, 200), (520, 193)])
+@pytest.mark.parametrize("precision", [None, "mixed"])
+def test_gemm_shapes_at_partial_tiles(rf, ora, monkeypatch, precision, k, u):
+    """Two leaves of k dense unknowns under a separator of u: update blocks of
+    u rows and K tails around the tile shapes' edges (and, for k > 512, the
+    update of the pivot columns themselves).  Every shape gives the same bits,
+    and pivots within n rounding errors of the working precision (times 8, the
+    condition of a matrix with row sums at most half its diagonal stays below
+    3) of the oracle's."""
+    n = 2 * k + u
+    rng = np.random.default_rng(1000 * k + u)
+    a = rng.standard_normal((n, n))
+    a[:k, k:2 * k] = a[k:2 * k, :k] = 0.0
+    a = (a + a.T) / 2
+    np.fill_diagonal(a, 0.0)
+    np.fill_diagonal(a, 2.0 * np.abs(a).sum(axis=1) + 1.0)
+    p = dense_problem(a)
+    print(f"case gemm shapes k={k} u={u} precision={precision}", flush=True)
+    _, _, d_o = ora.Handle.factor(p, want_d=True)
+    ds = []
+    for shape in ("0", "128x64", "128x128"):
+        monkeypatch.setenv("RUSTYFEM_AUTOTUNE", shape)
+        _, _, d = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
+        ds.append(d)
+    assert np.array_equal(ds[1], ds[0]) and np.array_equal(ds[2], ds[0])
+    eps = 2.0**-53 if precision is None else 2.0**-24
+    assert np.max(np.abs(ds[0] - d_o) / np.abs(d_o)) < 8 * n * eps
+
+
 @pytest.mark.parametrize("precision", [None, "mixed"])
 def test_lookahead_gives_identical_factor(rf, monkeypatch, precision):
     """The rest of each outer block's update runs on a second stream beside the
