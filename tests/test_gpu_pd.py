@@ -294,6 +294,32 @@ def test_inverse_and_chain_superblock_solves_agree(rf, monkeypatch):
     assert np.all(np.linalg.norm(p.rhs - a @ x_i, axis=0) / np.linalg.norm(p.rhs, axis=0) < 1e-12)
 
 
+@pytest.mark.parametrize("k", [1, 15, 17, 63, 65, 80, 129, 500, 513, 590])
+def test_superblock_inverse_at_partial_strips(rf, monkeypatch, k):
+    """One dense front of k pivots (more than 384 rows, or the solves of every
+    size through the super-block kernels): ragged 16-column strips, block rows
+    and super-blocks of the explicit inverse against the block chain.  The
+    matrix is diagonally dominant (condition below 3), so both solutions are
+    within a few n rounding errors of the exact one."""
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((k, k))
+    a = (a + a.T) / 2
+    np.fill_diagonal(a, 0.0)
+    np.fill_diagonal(a, 2.0 * np.abs(a).sum(axis=1) + 1.0)
+    p = dense_problem(a)
+    b = rng.standard_normal((k, 3))
+    print(f"case super-block strips k={k}", flush=True)
+    monkeypatch.setenv("RUSTYFEM_NO_SMALL_SOLVE", "1")
+    x = []
+    for chain in ("1", "0"):
+        monkeypatch.setenv("RUSTYFEM_SOLVE_CHAIN", chain)
+        h, _, _ = rf.Handle.factor(p, max_refine=0)
+        x.append(h.solve(b))
+    tol = 8 * (k + 8) * 2.0**-53
+    assert np.max(np.abs(x[1] - x[0])) <= tol * np.max(np.abs(x[0]))
+    assert np.max(np.abs(a @ x[1] - b)) <= tol * 3 * np.max(np.abs(b))
+
+
 @pytest.mark.parametrize("precision", [None, "mixed"])
 def test_gemm_register_layouts_agree(rf, monkeypatch, precision):
     """The Schur GEMM kernels (k_gemm, k_gemm_agpr, k_gemm_ilv, k_gemm_k64 and,
