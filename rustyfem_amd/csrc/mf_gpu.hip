@@ -286,10 +286,10 @@ __global__ __launch_bounds__(256) void k_panel(const FrontDesc* __restrict__ fd,
   __shared__ __attribute__((aligned(16))) double Vs[NB][NB + 2];        // L^-1 [col][row]
   __shared__ __attribute__((aligned(16))) double YY[2][KS][NB + 2];     // Ys, Y0; later scratch
   __shared__ double Xs[KS][NB + 2];   // L[r0 + i, k]
-  __shared__ double cbuf[NB], dd[NB];
+  __shared__ double dd[NB];
   double(*Ys)[NB + 2] = YY[0];        // L[j0 + q, k] d_k
   double(*Y0)[NB + 2] = YY[1];        // L[j0 + i, k]
-  static_assert(2 * KS * (NB + 2) >= 4 * 256, "the inverse's scratch fits in the update buffers");
+  static_assert(2 * KS * (NB + 2) >= kLdltScratch, "the inverse's scratch fits in the update buffers");
   M::acc_t cb[4], cr[4];
 #pragma unroll
   for (int bj = 0; bj < 4; ++bj) {
@@ -345,8 +345,13 @@ __global__ __launch_bounds__(256) void k_panel(const FrontDesc* __restrict__ fd,
   {
     const double orig = lane < jb ? adiag[static_cast<int64_t>(d.start) + t.j0 + lane] : 1.0;
     // the update buffers are free now: the inverse's scratch
-    block_ldlt_blk(Ad, Vs, &YY[0][0][0], cbuf, dd, jb, orig, static_cast<int64_t>(d.start) + t.j0,
+    block_ldlt_blk(Ad, Vs, &YY[0][0][0], dd, jb, orig, static_cast<int64_t>(d.start) + t.j0,
                    diag_tile ? err : nullptr);
+  }
+  // zero outside the lower triangle of jb x jb
+  for (int idx = tid; idx < NB * NB; idx += 256) {
+    const int q = idx / NB, i = idx % NB;
+    if (q >= jb || i >= jb || i < q) Vs[q][i] = 0.0;
   }
   __syncthreads();
   if (diag_tile) {

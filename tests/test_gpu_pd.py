@@ -320,6 +320,31 @@ def test_superblock_inverse_at_partial_strips(rf, monkeypatch, k):
     assert np.max(np.abs(a @ x[1] - b)) <= tol * 3 * np.max(np.abs(b))
 
 
+@pytest.mark.parametrize("k", [5, 16, 17, 33, 48, 49, 64, 100, 192, 193, 257, 300])
+@pytest.mark.parametrize("precision", [None, "mixed"])
+def test_pivot_steps_at_partial_blocks(rf, monkeypatch, precision, k):
+    """One dense front at the edges of the 16-column blocks, the 64-column
+    pivot blocks and the 256-column outer block: k_pdiag / k_prow against the
+    fused k_panel, which sums and eliminates in the same order (identical D,
+    solutions equal to rounding of the FP64 solves)."""
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((k, k))
+    a = (a + a.T) / 2
+    np.fill_diagonal(a, 0.0)
+    np.fill_diagonal(a, 2.0 * np.abs(a).sum(axis=1) + 1.0)
+    p = dense_problem(a)
+    b = rng.standard_normal((k, 2))
+    print(f"case pivot steps k={k} precision={precision}", flush=True)
+    out = []
+    for legacy in ("1", "0"):
+        monkeypatch.setenv("RUSTYFEM_LEGACY_PANEL", legacy)
+        h, err, d = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
+        assert err == -1
+        out.append((d, h.solve(b)))
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.max(np.abs(out[0][1] - out[1][1])) <= 8 * (k + 8) * 2.0**-53 * np.max(np.abs(out[0][1]))
+
+
 @pytest.mark.parametrize("precision", [None, "mixed"])
 def test_gemm_register_layouts_agree(rf, monkeypatch, precision):
     """The Schur GEMM kernels (k_gemm, k_gemm_agpr, k_gemm_ilv, k_gemm_k64 and,
