@@ -106,42 +106,17 @@ __device__ void inv3(const double m[3][3], double ji[3][3], double& det) {
   ji[2][2] = (m[0][0] * m[1][1] - m[0][1] * m[1][0]) * id;
 }
 
+// the sign of component c of hexahedron node i's natural coordinates (nodes
+// counterclockwise, bottom then top)
+__device__ inline double hex_sign(int i, int c) {
+  const int bit = c == 0 ? ((i + 1) >> 1) & 1 : c == 1 ? (i >> 1) & 1 : i >> 2;
+  return bit ? 1.0 : -1.0;
+}
+
 // dN/dx of integration point g and its weight; false when the Jacobian
 // determinant fails the reference's test.
 template <int KIND>
 __device__ bool ip_point(int g, const double (*x)[3], double thick, double (*dndx)[3], double& w);
-
-template <>
-__device__ bool ip_point<0>(int g, const double (*x)[3], double, double (*dndx)[3], double& w) {
-  // hex8_ip at the 2x2x2 points, xi fastest (src/elements/continuum3d.rs:39-84)
-  const double nat[8][3] = {{-1.0, -1.0, -1.0}, {1.0, -1.0, -1.0}, {1.0, 1.0, -1.0}, {-1.0, 1.0, -1.0},
-                            {-1.0, -1.0, 1.0},  {1.0, -1.0, 1.0},  {1.0, 1.0, 1.0},  {-1.0, 1.0, 1.0}};
-  const double p[3] = {(g & 1) ? G2 : -G2, (g & 2) ? G2 : -G2, (g & 4) ? G2 : -G2};
-  double dn[3][8];
-  for (int i = 0; i < 8; ++i) {
-    const double f0 = 1.0 + p[0] * nat[i][0], f1 = 1.0 + p[1] * nat[i][1], f2 = 1.0 + p[2] * nat[i][2];
-    dn[0][i] = 0.125 * nat[i][0] * f1 * f2;
-    dn[1][i] = 0.125 * nat[i][1] * f0 * f2;
-    dn[2][i] = 0.125 * nat[i][2] * f0 * f1;
-  }
-  double j[3][3];
-  for (int r = 0; r < 3; ++r)
-    for (int c = 0; c < 3; ++c) {
-      double s = 0.0;
-      for (int i = 0; i < 8; ++i) s = s + dn[r][i] * x[i][c];
-      j[r][c] = s;
-    }
-  double ji[3][3], det;
-  inv3(j, ji, det);
-  for (int i = 0; i < 8; ++i)
-    for (int c = 0; c < 3; ++c) {
-      double s = 0.0;
-      for (int r = 0; r < 3; ++r) s = s + ji[c][r] * dn[r][i];
-      dndx[i][c] = s;
-    }
-  w = det * 1.0;
-  return !(det <= 0.0);
-}
 
 template <>
 __device__ bool ip_point<1>(int, const double (*x)[3], double, double (*dndx)[3], double& w) {
@@ -264,7 +239,31 @@ struct Lds {
   double db[NG][NS][ND];  // D B
 };
 
+// The hexahedron's B and D B take few distinct values per point and node: with
+// n_k = dN/dx_k + corr_k and c_k = 0 + corr_k, a normal row holds n_k in its
+// own component and c_k in the others, a shear row plain derivatives.
+template <>
+struct Lds<0> {
+  double x[8][3];
+  double w[8];
+  double avg[24];
+  double bw[8][9][8];     // n_k w, c_k w, dN/dx_k w of [point][.][node]; first the dN/dxi, last the blocks to store
+  union {
+    double db[8][12][8];  // D B: normal rows (3 r + k), then mu dN/dx_k
+    struct {
+      double j[8][9];     // before: Jacobian of each point, derivatives
+      double dndx[8][8][3];
+    };
+  };
+};
+
 // Element stiffness blocks: 64-lane workgroups, 64 / NN^2 elements each.
+//
+// Bound by FP64 operations without contraction (a hexahedron: 624 in the last
+// loop alone) and by LDS reads, with few waves in flight (LDS).  64^3
+// hexahedra, 1,075 -> 739 us: 21 distinct values of B and D B per point and
+// node in LDS instead of 36, the Jacobians by all lanes instead of one lane
+// per point, the stores of an element consecutive.
 template <int KIND>
 __global__ __launch_bounds__(64) void k_elem(const int32_t* __restrict__ conn, const double* __restrict__ coords,
                                              const double* __restrict__ young, const double* __restrict__ pois,
@@ -281,7 +280,39 @@ __global__ __launch_bounds__(64) void k_elem(const int32_t* __restrict__ conn, c
   Lds<KIND>& s = S[slot];
   if (l < NN * 3) s.x[l / 3][l % 3] = coords[static_cast<int64_t>(conn[ec * NN + l / 3]) * 3 + l % 3];
   __syncthreads();
-  if (l < NG) {
+  if constexpr (KIND == 0) {
+    // hex8_ip at the 2x2x2 points, xi fastest (src/elements/continuum3d.rs:39-84),
+    // lane 8 g + i at point g and node i: dN/dxi, then Jacobian entries i and 8
+    const int g = l >> 3, i = l & 7;
+    const double p0 = (g & 1) ? G2 : -G2, p1 = (g & 2) ? G2 : -G2, p2 = (g & 4) ? G2 : -G2;
+    const double n0 = hex_sign(i, 0), n1 = hex_sign(i, 1), n2 = hex_sign(i, 2);
+    const double f0 = 1.0 + p0 * n0, f1 = 1.0 + p1 * n1, f2 = 1.0 + p2 * n2;
+    const double dn[3] = {0.125 * n0 * f1 * f2, 0.125 * n1 * f0 * f2, 0.125 * n2 * f0 * f1};
+    for (int r = 0; r < 3; ++r) s.bw[g][r][i] = dn[r];
+    __syncthreads();
+    auto entry = [&](int rc) {
+      const int r = rc / 3, c = rc % 3;
+      double acc = 0.0;
+      for (int q = 0; q < 8; ++q) acc = acc + s.bw[g][r][q] * s.x[q][c];
+      s.j[g][rc] = acc;
+    };
+    entry(i);
+    if (i == 0) entry(8);
+    __syncthreads();
+    double j[3][3], ji[3][3], det;
+    for (int r = 0; r < 3; ++r)
+      for (int c = 0; c < 3; ++c) j[r][c] = s.j[g][3 * r + c];
+    inv3(j, ji, det);
+    for (int c = 0; c < 3; ++c) {
+      double acc = 0.0;
+      for (int r = 0; r < 3; ++r) acc = acc + ji[c][r] * dn[r];
+      s.dndx[g][i][c] = acc;
+    }
+    if (i == 0) {
+      s.w[g] = det * 1.0;
+      if (det <= 0.0 && live) atomicMin(bad, static_cast<unsigned long long>(e));
+    }
+  } else if (l < NG) {
     double w;
     const bool ok = ip_point<KIND>(l, s.x, thick[ec], s.dndx[l], w);
     s.w[l] = w;
@@ -299,7 +330,30 @@ __global__ __launch_bounds__(64) void k_elem(const int32_t* __restrict__ conn, c
     s.avg[l] = acc / wsum;
   }
   __syncthreads();
-  {
+  if constexpr (KIND == 0) {
+    const Dmat<KIND> D(young[ec], pois[ec]);
+    const int g = l >> 3, i = l & 7;
+    const double wg = s.w[g];
+    const double dx[3] = {s.dndx[g][i][0], s.dndx[g][i][1], s.dndx[g][i][2]};
+    __syncthreads();  // db overwrites the derivatives
+    for (int k = 0; k < 3; ++k) {
+      const double d = dx[k];
+      const double corr = (s.avg[3 * i + k] - d) / 3.0;
+      const double nk = d + corr, ck = 0.0 + corr;
+      s.bw[g][k][i] = nk * wg;
+      s.bw[g][3 + k][i] = ck * wg;
+      s.bw[g][6 + k][i] = d * wg;
+      for (int r = 0; r < 3; ++r) {
+        double acc = 0.0;
+        for (int m = 0; m < 3; ++m)
+          if (D.v[r][m] != 0.0) acc = acc + D.v[r][m] * (m == k ? nk : ck);
+        s.db[g][3 * r + k][i] = acc;
+      }
+      double acc = 0.0;
+      if (D.v[3][3] != 0.0) acc = acc + D.v[3][3] * d;
+      s.db[g][9 + k][i] = acc;
+    }
+  } else {
     const Dmat<KIND> D(young[ec], pois[ec]);
     for (int q = l; q < NG * NN; q += LPE) {
       const int g = q / NN, i = q % NN;
@@ -330,20 +384,45 @@ __global__ __launch_bounds__(64) void k_elem(const int32_t* __restrict__ conn, c
   double k[DIM][DIM];
   for (int ki = 0; ki < DIM; ++ki)
     for (int kj = 0; kj < DIM; ++kj) k[ki][kj] = 0.0;
-  for (int g = 0; g < NG; ++g) {
+  if constexpr (KIND == 0) {
+    for (int g = 0; g < NG; ++g) {
+      double bv[9], dv[12];
 #pragma unroll
-    for (int r = 0; r < NS; ++r) {
-      double bv[DIM], dv[DIM];
+      for (int q = 0; q < 9; ++q) bv[q] = s.bw[g][q][a];
 #pragma unroll
-      for (int q = 0; q < DIM; ++q) {
-        bv[q] = nz_b<KIND>(r, q) ? s.bw[g][r][DIM * a + q] : 0.0;
-        dv[q] = nz_db<KIND>(r, q) ? s.db[g][r][DIM * bn + q] : 0.0;
+      for (int q = 0; q < 12; ++q) dv[q] = s.db[g][q][bn];
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int ki = 0; ki < 3; ++ki)
+#pragma unroll
+          for (int kj = 0; kj < 3; ++kj) k[ki][kj] = k[ki][kj] + bv[ki == r ? ki : 3 + ki] * dv[3 * r + kj];
+      // shear row of the components (p, q): dN/dx_q in p, dN/dx_p in q
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        const int p = r == 2 ? 1 : 0, q = r == 0 ? 1 : 2;
+        k[p][p] = k[p][p] + bv[6 + q] * dv[9 + q];
+        k[p][q] = k[p][q] + bv[6 + q] * dv[9 + p];
+        k[q][p] = k[q][p] + bv[6 + p] * dv[9 + q];
+        k[q][q] = k[q][q] + bv[6 + p] * dv[9 + p];
       }
+    }
+  } else {
+    for (int g = 0; g < NG; ++g) {
 #pragma unroll
-      for (int ki = 0; ki < DIM; ++ki)
+      for (int r = 0; r < NS; ++r) {
+        double bv[DIM], dv[DIM];
 #pragma unroll
-        for (int kj = 0; kj < DIM; ++kj)
-          if (nz_b<KIND>(r, ki) && nz_db<KIND>(r, kj)) k[ki][kj] = k[ki][kj] + bv[ki] * dv[kj];
+        for (int q = 0; q < DIM; ++q) {
+          bv[q] = nz_b<KIND>(r, q) ? s.bw[g][r][DIM * a + q] : 0.0;
+          dv[q] = nz_db<KIND>(r, q) ? s.db[g][r][DIM * bn + q] : 0.0;
+        }
+#pragma unroll
+        for (int ki = 0; ki < DIM; ++ki)
+#pragma unroll
+          for (int kj = 0; kj < DIM; ++kj)
+            if (nz_b<KIND>(r, ki) && nz_db<KIND>(r, kj)) k[ki][kj] = k[ki][kj] + bv[ki] * dv[kj];
+      }
     }
   }
   // the transposed block from lane (b, a)
@@ -353,8 +432,22 @@ __global__ __launch_bounds__(64) void k_elem(const int32_t* __restrict__ conn, c
   for (int ki = 0; ki < DIM; ++ki)
 #pragma unroll
     for (int kj = 0; kj < DIM; ++kj) kt[kj][ki] = __shfl(k[ki][kj], partner, 64);
-  if (live && a <= bn) {
-    const int pair = a * NN - a * (a - 1) / 2 + (bn - a);
+  const int pair = a * NN - a * (a - 1) / 2 + (bn - a);
+  if constexpr (KIND == 0) {
+    // the element's 324 values leave as consecutive stores
+    double* o = &s.bw[0][0][0];
+    static_assert(sizeof(s.bw) >= NPAIR * DIM * DIM * sizeof(double), "the blocks fit");
+    __syncthreads();
+    if (a <= bn) {
+#pragma unroll
+      for (int ki = 0; ki < DIM; ++ki)
+#pragma unroll
+        for (int kj = 0; kj < DIM; ++kj) o[pair * (DIM * DIM) + ki * DIM + kj] = 0.5 * (k[ki][kj] + kt[ki][kj]);
+    }
+    __syncthreads();
+    if (live)
+      for (int q = l; q < NPAIR * DIM * DIM; q += LPE) ke[ec * (NPAIR * DIM * DIM) + q] = o[q];
+  } else if (live && a <= bn) {
     double* o = ke + (ec * NPAIR + pair) * (DIM * DIM);
 #pragma unroll
     for (int ki = 0; ki < DIM; ++ki)
@@ -364,6 +457,11 @@ __global__ __launch_bounds__(64) void k_elem(const int32_t* __restrict__ conn, c
 }
 
 // out[p] = sum of the element-matrix entries of entry p, in list order, from zero
+//
+// Four list entries at a time, so that their loads overlap: bound by the bytes
+// it moves and the lines it touches instead of by two dependent loads per
+// addition.  64^3 hexahedra: 987 -> 840 us (a contiguous run of entries for
+// each XCD's L2: 877).
 __global__ __launch_bounds__(256) void k_gather_sum(const uint32_t* __restrict__ off, const uint32_t* __restrict__ src,
                                                     const double* __restrict__ ke, int64_t nout,
                                                     double* __restrict__ out) {
@@ -371,7 +469,14 @@ __global__ __launch_bounds__(256) void k_gather_sum(const uint32_t* __restrict__
   if (p >= nout) return;
   double s = 0.0;
   const uint32_t k1 = off[p + 1];
-  for (uint32_t k = off[p]; k < k1; ++k) s = s + ke[src[k]];
+  for (uint32_t k = off[p]; k < k1; k += 4) {
+    double v[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) v[u] = ke[src[min(k + u, k1 - 1)]];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u)
+      if (k + u < k1) s = s + v[u];
+  }
   out[p] = s;
 }
 

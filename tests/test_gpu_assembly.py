@@ -107,6 +107,18 @@ def test_matches_structured_assembly(rf):
     np.testing.assert_allclose(got, p.data, rtol=0, atol=1e-12 * np.abs(p.data).max())
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 1, 1), (3, 5, 2)])
+def test_hexahedra_without_lateral_coupling(rf, ora, shape):
+    """nu = 0 in some elements (the normal rows of D are diagonal: the
+    reference skips their zeros) in meshes whose entries take 1 to 8 elements
+    (the gather goes by fours): the oracle's bits."""
+    p, conn, coords, eq = perturbed_hex(*shape, seed=11, amp=0.05)
+    young, nu, _ = materials(conn.shape[0], 12)
+    nu[::2] = 0.0
+    print(f"case hexahedra nu=0 {shape}", flush=True)
+    check_bits(rf, ora, "C3D8", conn, coords, eq, p.n, young, nu, None)
+
+
 def test_collapsed_hexahedra(rf, ora):
     """Wedges meshed as hexahedra with a repeated node: the reference adds
     every local pair, the repeated ones included, in its loop order."""
