@@ -1,4 +1,4 @@
-// Sums and maxima across the lanes of a DPP row, lane reads, and a workgroup
+// Sums across the lanes of a DPP row, lane reads, and a workgroup
 // barrier for LDS alone (gfx950).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -23,16 +23,6 @@ __device__ __forceinline__ double row16_sum(double v) {
   v += dpp_d<0x4E>(v);
   v += dpp_d<0x124>(v);
   v += dpp_d<0x128>(v);
-  return v;
-}
-
-// maximum over the 16 lanes of a DPP row (fmax: a NaN is passed over), in
-// every lane of the row
-__device__ __forceinline__ double row16_max(double v) {
-  v = fmax(v, dpp_d<0xB1>(v));
-  v = fmax(v, dpp_d<0x4E>(v));
-  v = fmax(v, dpp_d<0x124>(v));
-  v = fmax(v, dpp_d<0x128>(v));
   return v;
 }
 
