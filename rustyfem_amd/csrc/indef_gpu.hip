@@ -379,7 +379,13 @@ __device__ __forceinline__ void put_piv(const IRec& R, int p, double d, double e
 // and decisions are identical.  When a candidate fails, the columns are
 // brought up to date and that pivot goes through the full search with
 // interchanges and 2 x 2 pivots (ichoose, iswap, ielim1/2); so does everything
-// in a front with more than NT RPT rows or a widened block.
+// in a front with more than NT RPT rows or a widened block.  After two segments
+// in a row that took no pivot every pivot goes there until one passes in place
+// again: where most need an interchange or a 2 x 2 block, a trial per pivot and
+// the panel written back after it cost more than the register path saves
+// (refactorization, step by step / a trial per pivot / this: bipartite 24^3
+// grid with a zero diagonal 19.1 / 22.9 / 17.4 ms, 16^3 grid with a multiplier
+// of zero diagonal per node 22.5 / 25.4 / 21.6 ms).
 //
 // Bound by the instructions its one compute unit issues (16 waves: about 100
 // of them per pivot and wave).  32^3 shifted Laplacian, 41 launches per
@@ -458,8 +464,9 @@ __global__ __launch_bounds__(NT) void k_ipanel(const IRec* __restrict__ recs, IS
       }
     }
   };
+  int miss = 0;  // segments in a row that ended at their first candidate
   while (p < b1) {
-    if (fast) {
+    if (fast && miss < 2) {
       const int seg = p;  // every panel column is up to date with the pivots before seg
       bool stop = false;
       if (tid < b1 - seg) ssc[seg - p0 + tid] = scale[R.fs[seg + tid]];
@@ -527,6 +534,9 @@ __global__ __launch_bounds__(NT) void k_ipanel(const IRec* __restrict__ recs, IS
           c0 += cw;
         }
       }
+      miss = p == seg ? miss + 1 : 0;
+      // (no pivot taken: the columns in memory are up to date)
+      if (p == seg) c0 = b1;
       for (; c0 < b1; c0 += CB) {
         const int cw = min(CB, b1 - c0);
         double v[RPT][CB];
@@ -543,6 +553,7 @@ __global__ __launch_bounds__(NT) void k_ipanel(const IRec* __restrict__ recs, IS
     int j = 0, r = 0;
     const int kd = ichoose<NT>(G, m, p, b1, R.fs, scale, thr, j, r, red, redk);
     if (kd == 1) {
+      if (j == p) miss = 0;
       iswap<NT>(G, m, kf, R.fs, p, j);
       const double dp = ielim1<NT>(G, m, p, b1, sh.wl);
       if (tid == 0) put_piv(R, p, dp, 0.0, 1);

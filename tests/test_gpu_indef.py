@@ -176,6 +176,44 @@ def test_dense_fronts_around_the_panel_sizes(rf, ora, n, weak):
     assert relres(p, h.solve(b), b) < 1e-9
 
 
+@pytest.mark.parametrize("case", ["bipartite8", "bipartite10", "multiplier6", "stretches150", "stretches700"])
+def test_candidates_that_fail_in_place(rf, ora, case):
+    """Matrices where most candidates fail the threshold test in place, so that
+    the panel kernel leaves its register path: zero diagonals throughout, a
+    zero-diagonal multiplier beside an ordinary unknown at every node, and
+    stretches of either kind inside one pivot block (the path is left and taken
+    up again)."""
+    import scipy.sparse as sp
+    print(f"case in-place failures {case}", flush=True)
+    kind, n = case.rstrip("0123456789"), int(case.lstrip("abcdefghijklmnopqrstuvwxyz"))
+    if kind == "bipartite":
+        p = bipartite_grid(n, 2, 0.0)
+    elif kind == "multiplier":
+        g = laplacian3d(n)
+        a = sp.kron(csc(g), np.diag([1.0, 0.0])) + sp.kron(csc(bipartite_grid(n, 3, 1.0)), np.eye(2)[::-1])
+        pattern = sp.kron(csc(g), np.ones((2, 2))).tocoo()  # the zero diagonal is stored
+        order = np.lexsort((pattern.row, pattern.col))
+        vals = np.asarray(a.tocsr()[pattern.row, pattern.col]).ravel()
+        ptr = np.concatenate([[0], np.cumsum(np.bincount(pattern.col, minlength=2 * g.n))])
+        p = SimpleNamespace(n=2 * g.n, nn=g.n, loc=np.repeat(np.arange(g.n, dtype=np.int64), 2), coords=g.coords,
+                            indptr=ptr.astype(np.int64), indices=pattern.row[order].astype(np.int64), data=vals[order])
+    else:
+        rng = np.random.default_rng(n)
+        a = rng.standard_normal((n, n))
+        a = a + a.T
+        weak = (np.arange(n) // 11) % 2 == 0
+        np.fill_diagonal(a, np.where(weak, 0.0, 4.0 * n))
+        p = dense_problem(a)
+    h, err, ine = rf.Handle.factor_indef(p)
+    assert h is not None, rf.last_error()
+    ho, _, ineo = ora.Handle.factor_indef(p)
+    assert list(ine) == list(ineo)
+    assert_same_factor(h, ho)
+    assert h.factor_stats()[4] > 0
+    b = np.cos(np.arange(p.n) * 0.3)
+    assert relres(p, h.solve(b), b) < 1e-9
+
+
 def test_delays_reach_many_levels(rf, ora):
     """A larger strongly indefinite grid with delays at several levels."""
     p = bipartite_grid(10, 3, 1e-3)
