@@ -18,7 +18,7 @@ LIB = os.path.join(HERE, "librustyfem_ffi.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
-HOST_SOURCES = ["symbolic.cpp", "mf_plan.cpp", "plan_check.cpp", "amg_setup.cpp", "ffi.cpp"]
+HOST_SOURCES = ["symbolic.cpp", "mf_plan.cpp", "plan_check.cpp", "ic0_plan.cpp", "amg_setup.cpp", "ffi.cpp"]
 HIP_SOURCES = ["mf_gpu.hip", "indef_gpu.hip", "pcg_gpu.hip", "mpnn_gpu.hip", "ic0_gpu.hip", "eigen_gpu.hip",
                "assembly_gpu.hip"]
 # kernels that restate a CPU operation order entry by entry: no contraction

@@ -30,11 +30,14 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <future>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "ic0.hpp"
+#include "ic0_plan.hpp"
 #include "lane_ops.hpp"
 
 namespace rf {
@@ -69,6 +72,11 @@ struct Dev {
     p = nullptr;
     n = count;
     ICHK(hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)));
+  }
+  void free() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    n = 0;
   }
   void put(const std::vector<T>& v) {
     alloc(v.size());
@@ -131,14 +139,11 @@ __global__ __launch_bounds__(64) void k_ic0_factor(int64_t lb, const int32_t* __
   }
 }
 
-// dst[q] = src[tmap[q]] (0 where the map is negative): the factor's values in
-// the order of U's rows, or of a sweep's stream
+// dst[q] = src[tmap[q]]: the factor's values in the order of U's rows
 __global__ __launch_bounds__(TB) void k_gather(int64_t n, const int64_t* __restrict__ tmap,
                                                const double* __restrict__ src, double* __restrict__ dst) {
-  for (int64_t q = static_cast<int64_t>(blockIdx.x) * TB + threadIdx.x; q < n; q += static_cast<int64_t>(gridDim.x) * TB) {
-    const int64_t t = tmap[q];
-    dst[q] = t >= 0 ? src[t] : 0.0;
-  }
+  for (int64_t q = static_cast<int64_t>(blockIdx.x) * TB + threadIdx.x; q < n; q += static_cast<int64_t>(gridDim.x) * TB)
+    dst[q] = src[tmap[q]];
 }
 
 // y_i = r_i - sum_j L_ij y_j for the rows list[lb, le)
@@ -184,35 +189,6 @@ __global__ __launch_bounds__(TB) void k_ic0_div(int64_t n, const double* __restr
 }
 
 // ------------------------------------------------------- one-workgroup sweep
-
-constexpr int SWT = 512;           // threads of the sweep's workgroup
-constexpr int SWG = 8;             // lanes per group
-constexpr int SWS = SWT / SWG;     // groups per round
-constexpr int SWD = 3;             // rounds whose records are in flight
-constexpr int RING = 20000;        // solution values kept in LDS (160 KB with the entry that stays 0)
-// rounds of R values per slot that the ring holds
-constexpr int ring_rounds(int R) { return RING / (SWS * R); }
-
-// A round's slot holds one group of up to R rows: a word per slot with the
-// group's first row (its others follow in the sweep's direction), the number
-// of its rows, and two flags.
-constexpr uint32_t SW_LAST = 1;    // the last round of its level (in every slot of the round)
-constexpr uint32_t SW_TAIL = 2;    // columns beyond the record
-__host__ __device__ constexpr uint32_t slot_word(int64_t row, int cnt, uint32_t flags) {
-  return static_cast<uint32_t>(row) << 4 | static_cast<uint32_t>(cnt) << 2 | flags;
-}
-
-// A thread's record of one round: NC columns (LDS byte offsets of their values
-// in the ring), the slot's word SWD rounds later, the columns' R factor
-// values each, and, for row r < R of the group in lane r, the coefficients of
-// t_0 .. t_{R-2} in x_r (the inverse of the group's unit triangle).  Stored in
-// 16-byte granules interleaved over the wave's lanes.
-template <int R, int NC>
-struct SweepRecord {
-  static constexpr int NI = NC + 1, ND = NC * R + R - 1;
-  static constexpr int GI = (NI + 3) / 4, GD = (ND + 1) / 2;  // granules of words, of doubles
-  static constexpr int GRANULES = GI + GD;
-};
 
 // sum over 8 consecutive lanes, in every lane: quad_perm [1,0,3,2], quad_perm
 // [2,3,0,1], row_half_mirror
@@ -361,245 +337,84 @@ __global__ __launch_bounds__(SWT) void k_ic0_sweep(int rounds, const uint32_t* _
   }
 }
 
-// the factor values of the records: double q of the stream is lval[map[q]], 0
-// where the map is negative (map given for the doubles in stream order)
-__global__ __launch_bounds__(TB) void k_ic0_records(int64_t n, const int32_t* __restrict__ map,
-                                                    const int64_t* __restrict__ place,
-                                                    const double* __restrict__ lval, double* __restrict__ rec) {
-  const int64_t q = static_cast<int64_t>(blockIdx.x) * TB + threadIdx.x;
-  if (q < n) rec[place[q]] = lval[map[q]];
-}
-
-// coefficients of a group's rows: x_1 = t_1 - l_10 t_0, x_2 = t_2 + (l_21 l_10
-// - l_20) t_0 - l_21 t_1; `at` holds their places in the stream
-struct SweepCoef { int32_t l10, l20, l21, pad; int64_t at[3]; };
-__global__ __launch_bounds__(TB) void k_ic0_coefs(int64_t n, const SweepCoef* __restrict__ c,
-                                                  const double* __restrict__ lval, double* __restrict__ rec) {
-  const int64_t q = static_cast<int64_t>(blockIdx.x) * TB + threadIdx.x;
-  if (q >= n) return;
-  const SweepCoef s = c[q];
-  const double l10 = lval[s.l10];
-  rec[s.at[0]] = -l10;
-  if (s.l20 >= 0) {
-    const double l20 = lval[s.l20], l21 = lval[s.l21];
-    rec[s.at[1]] = l21 * l10 - l20;
-    rec[s.at[2]] = -l21;
-  }
-}
-
-// rows grouped by level: list (rows in increasing order within a level) and
-// the level offsets
-void by_level(const std::vector<int32_t>& lev, int32_t nlev, std::vector<int32_t>& list, std::vector<int64_t>& off) {
-  off.assign(static_cast<size_t>(nlev) + 1, 0);
-  for (int32_t l : lev) ++off[l + 1];
-  for (int32_t l = 0; l < nlev; ++l) off[l + 1] += off[l];
-  list.resize(lev.size());
-  std::vector<int64_t> pos(off.begin(), off.end() - 1);
-  for (size_t i = 0; i < lev.size(); ++i) list[pos[lev[i]]++] = static_cast<int32_t>(i);
-}
-
-// The schedule and stream of one sweep over the strictly triangular rows
-// (ptr, idx: columns sorted; forward: columns below the row, dir = 1;
-// backward: above it, dir = -1).  src[p] is the factor value of entry p.
-struct SweepPlan {
-  int R = 0;                    // rows per group (1, 2 or 3); 0: not possible
-  int NC = 0;                   // columns per lane in a record (2, 3 or 5)
-  int64_t levels = 0, rounds = 0;
-  std::vector<uint32_t> word0;  // the slots' words of the first SWD rounds
-  std::vector<int32_t> rec;     // the records' words (the doubles' places 0)
-  std::vector<int32_t> vmap;    // factor values and their places among the records' doubles
-  std::vector<int64_t> place;
-  std::vector<SweepCoef> coef;
-  std::vector<int32_t> tptr, tcol, tmap;  // the tails: slots' offsets, ring offsets, R factor values (-1: 0) each
-};
-
-template <int R, int NC>
-void fill_records(SweepPlan& S, const std::vector<int64_t>& ptr, const std::vector<int32_t>& idx,
-                  const std::vector<int64_t>* src, int dir, const std::vector<int32_t>& first,
-                  const std::vector<int32_t>& cnt, const std::vector<int32_t>& slot_group,
-                  const std::vector<int32_t>& slot_of, const std::vector<int32_t>& group_of,
-                  const std::vector<uint32_t>& words) {
+// The records (and tails) of a sweep from its schedule: lane by lane of every
+// slot, the ring places of its columns and the factor's values.  map: the place
+// of entry p of (ptr, idx) in lval (null: p).  The host only lays out the
+// schedule, in two threads beside the factorization: setup of the 20^3 block
+// 92 ms with the records built entry by entry on the host, 67 ms so (66 without
+// sweeps); plate of 500 x 200 quadrilaterals 160, 96 and 95 ms.
+template <int R, int NC, int DIR>
+__global__ __launch_bounds__(TB) void k_ic0_records(int64_t slots, const uint32_t* __restrict__ words,
+                                                    const int32_t* __restrict__ ring, const int32_t* __restrict__ tptr,
+                                                    const int64_t* __restrict__ ptr, const int32_t* __restrict__ idx,
+                                                    const int64_t* __restrict__ map, const double* __restrict__ lval,
+                                                    v4i* __restrict__ rec, int32_t* __restrict__ tcol,
+                                                    double* __restrict__ tval) {
   using Rec = SweepRecord<R, NC>;
-  auto entry = [&](int64_t p) { return static_cast<int32_t>(src ? (*src)[p] : p); };
-  const int64_t waves = S.rounds + SWD, per = static_cast<int64_t>(SWT / 64) * Rec::GRANULES * 64 * 4;
-  S.rec.assign(static_cast<size_t>(waves * per), 0);
-  // word w of the lane of (round, slot): granule w / 4
-  auto word_at = [&](int64_t q, int lane, int w) {
-    const int64_t t = q / SWS, th = (q % SWS) * SWG + lane;
-    return ((t * (SWT / 64) + th / 64) * Rec::GRANULES + w / 4) * 256 + (th % 64) * 4 + w % 4;
-  };
-  auto double_at = [&](int64_t q, int lane, int d) { return word_at(q, lane, 4 * Rec::GI + 2 * d) / 2; };
-  constexpr int32_t zero = ring_rounds(R) * SWS * R * 8;
-  S.tptr.assign(static_cast<size_t>(waves * SWS) + 1, 0);
-  S.vmap.reserve(idx.size());
-  S.place.reserve(idx.size());
-  for (int64_t q = 0; q < waves * SWS; ++q) {
-    S.tptr[q] = static_cast<int32_t>(S.tcol.size());
-    const int64_t next = q + static_cast<int64_t>(SWD) * SWS;
-    const uint32_t nw = next < static_cast<int64_t>(words.size()) ? words[next] : 0;
-    for (int lane = 0; lane < SWG; ++lane) {
-      for (int c = 0; c < NC; ++c) S.rec[word_at(q, lane, c)] = zero;
-      S.rec[word_at(q, lane, NC)] = static_cast<int32_t>(nw);
-    }
-    const int32_t g = q < static_cast<int64_t>(slot_group.size()) ? slot_group[q] : -1;
-    if (g < 0) continue;
-    const int64_t f = first[g];
-    const int c = cnt[g];
-    const int64_t k = ptr[f + 1] - ptr[f];
-    int64_t rowp[R];  // row r's entries of the shared columns
-    for (int r = 0; r < R; ++r) rowp[r] = ptr[f + dir * std::min(r, c - 1)] + (dir > 0 ? 0 : std::min(r, c - 1));
-    for (int64_t j = 0; j < k; ++j) {
-      const int32_t col = idx[ptr[f] + j], cg = group_of[col];
-      const int64_t cq = slot_of[cg];
-      const int32_t at = static_cast<int32_t>(
-          ((cq / SWS % ring_rounds(R)) * SWS * R + (cq % SWS) * R + dir * (col - first[cg])) * 8);
-      if (j < SWG * NC) {
-        const int lane = static_cast<int>(j % SWG), cc = static_cast<int>(j / SWG);
-        S.rec[word_at(q, lane, cc)] = at;
-        for (int r = 0; r < c; ++r) {
-          S.vmap.push_back(entry(rowp[r] + j));
-          S.place.push_back(double_at(q, lane, cc * R + r));
-        }
-      } else {
-        S.tcol.push_back(at);
-        for (int r = 0; r < R; ++r) S.tmap.push_back(r < c ? entry(rowp[r] + j) : -1);
+  const int64_t th = static_cast<int64_t>(blockIdx.x) * TB + threadIdx.x;
+  const int64_t q = th / SWG;
+  const int lane = static_cast<int>(th % SWG);
+  if (q >= slots) return;
+  const uint32_t word = words[q];
+  const int64_t f = slot_row(word);
+  const int cnt = slot_rows(word);
+  const int64_t p0 = ptr[f], k = cnt ? ptr[f + 1] - p0 : 0;
+  auto value = [&](int64_t p) { return lval[map ? map[p] : p]; };
+  int64_t rowp[R];  // row r's entries of the shared columns
+#pragma unroll
+  for (int r = 0; r < R; ++r) rowp[r] = ptr[r < cnt ? f + DIR * r : f] + (DIR > 0 ? 0 : r);
+  int32_t w[4 * Rec::GI] = {};
+  double d[2 * Rec::GD] = {};
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int64_t j = c * SWG + lane;
+    w[c] = j < k ? ring[idx[p0 + j]] : ring_rounds(R) * SWS * R * 8;
+#pragma unroll
+    for (int r = 0; r < R; ++r) d[c * R + r] = (j < k && r < cnt) ? value(rowp[r] + j) : 0.0;
+  }
+  w[NC] = static_cast<int32_t>(words[q + SWD * SWS]);
+  // the coefficients of the group's rows: x_1 = t_1 - l_10 t_0,
+  // x_2 = t_2 + (l_21 l_10 - l_20) t_0 - l_21 t_1
+  if constexpr (R > 1) {
+    // row r's entry in the group's row m (m < r)
+    auto own = [&](int r, int m) { return value(ptr[f + DIR * r] + (DIR > 0 ? k + m : r - 1 - m)); };
+    if (lane == 1 && cnt > 1) d[NC * R] = -own(1, 0);
+    if constexpr (R > 2) {
+      if (lane == 2 && cnt > 2) {
+        const double l21 = own(2, 1);
+        d[NC * R] = l21 * own(1, 0) - own(2, 0);
+        d[NC * R + 1] = -l21;
       }
-    }
-    if (c > 1) {
-      // row r's entry in the group's row m (m < r)
-      auto own = [&](int r, int m) {
-        const int64_t row = f + dir * r;
-        return entry(dir > 0 ? ptr[row] + k + m : ptr[row] + (r - 1 - m));
-      };
-      SweepCoef co{own(1, 0), -1, -1, 0, {double_at(q, 1, NC * R), 0, 0}};
-      if (c > 2) {
-        co.l20 = own(2, 0);
-        co.l21 = own(2, 1);
-        co.at[1] = double_at(q, 2, NC * R);
-        co.at[2] = double_at(q, 2, NC * R + 1);
-      }
-      S.coef.push_back(co);
     }
   }
-  S.tptr.back() = static_cast<int32_t>(S.tcol.size());
+  const int64_t in = th % SWT;
+  v4i* o = rec + ((q / SWS) * (SWT / 64) + in / 64) * (Rec::GRANULES * 64) + in % 64;
+#pragma unroll
+  for (int g = 0; g < Rec::GI; ++g) o[64 * g] = v4i{w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3]};
+#pragma unroll
+  for (int g = 0; g < Rec::GD; ++g)
+    o[64 * (Rec::GI + g)] = __builtin_bit_cast(v4i, d2{d[2 * g], d[2 * g + 1]});
+  if (word & SW_TAIL) {
+    const int64_t t0 = static_cast<int64_t>(tptr[q]) - SWG * NC;
+    for (int64_t j = SWG * NC + lane; j < k; j += SWG) {
+      tcol[t0 + j] = ring[idx[p0 + j]];
+#pragma unroll
+      for (int r = 0; r < R; ++r) tval[(t0 + j) * R + r] = r < cnt ? value(rowp[r] + j) : 0.0;
+    }
+  }
 }
 
-// One workgroup's sweep against a launch per row level, measured per
-// application on C3D8 blocks (both sweeps, row levels in brackets):
-//   8^3 (168) 138 against 896 us, 16^3 (336) 319 / 2,205, 24^3 (504) 702 / 4,386,
-//   32^3 (672) 1,383 / 5,258, 40^3 (840) 2,551 / 7,099, 56^3 (1,176) 10,932 / 11,095.
-// That is about 0.2 us per level and 0.9 us per round of 64 groups, 1.7 us per
-// round where the records exceed the Infinity Cache and come from HBM,
-// against 3.4 us per launch (more where a level has thousands of rows).
-bool sweep_pays(int64_t levels, int64_t rounds, int R, int NC) {
-  const double bytes = static_cast<double>(rounds) * SWT * 8 * (NC * R + R + (NC + 1) / 2 + 1);
-  return 0.2 * static_cast<double>(levels) + (bytes < 128e6 ? 0.9 : 1.7) * static_cast<double>(rounds) <
-         3.4 * R * static_cast<double>(levels);
-}
-
-SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vector<int32_t>& idx,
-                     const std::vector<int64_t>* src, int dir) {
-  SweepPlan S;
-  if (n >= (int64_t(1) << 28) || idx.size() >= (size_t(1) << 30)) return S;
-  // groups: consecutive rows (in elimination order) whose columns are the
-  // first row's columns and the rows of the group before them
-  std::vector<int32_t> first, cnt;  // first row and rows of every group, in elimination order
-  auto build = [&](int R) {
-    first.clear();
-    cnt.clear();
-    for (int64_t e = 0; e < n; ++e) {
-      const int64_t row = dir > 0 ? e : n - 1 - e;
-      bool join = false;
-      if (!first.empty() && cnt.back() < R) {
-        const int64_t f = first.back();
-        const int c = cnt.back();
-        const int64_t k = ptr[f + 1] - ptr[f];
-        if (ptr[row + 1] - ptr[row] == k + c) {
-          // the group's rows come last (forward) or first (backward)
-          const int32_t* own = idx.data() + ptr[row] + (dir > 0 ? k : 0);
-          const int32_t* ext = idx.data() + ptr[row] + (dir > 0 ? 0 : c);
-          const int32_t lo = static_cast<int32_t>(dir > 0 ? f : row + 1);
-          join = std::equal(ext, ext + k, idx.data() + ptr[f]);
-          for (int q = 0; join && q < c; ++q) join = own[q] == lo + q;
-        }
-      }
-      if (join) {
-        ++cnt.back();
-      } else {
-        first.push_back(static_cast<int32_t>(row));
-        cnt.push_back(1);
-      }
-    }
+// f(R, NC) for a plan's constants
+template <typename F>
+void with_constants(int R, int NC, F f) {
+  auto nc = [&](auto r) {
+    if (NC == 2) f(r, std::integral_constant<int, 2>());
+    else if (NC == 3) f(r, std::integral_constant<int, 3>());
+    else f(r, std::integral_constant<int, 5>());
   };
-  // the largest group size that wastes at most a quarter of its rows
-  int R = 3;
-  for (; R > 1; --R) {
-    build(R);
-    if (static_cast<double>(n) >= 0.75 * R * static_cast<double>(first.size())) break;
-  }
-  if (R == 1) build(1);
-  const int64_t ng = static_cast<int64_t>(first.size());
-  std::vector<int32_t> group_of(n), lev(ng, 0);
-  for (int64_t g = 0; g < ng; ++g)
-    for (int c = 0; c < cnt[g]; ++c) group_of[first[g] + dir * c] = static_cast<int32_t>(g);
-  int32_t nlev = ng ? 1 : 0;
-  for (int64_t g = 0; g < ng; ++g) {
-    int32_t l = 0;
-    for (int64_t p = ptr[first[g]]; p < ptr[first[g] + 1]; ++p) l = std::max(l, lev[group_of[idx[p]]] + 1);
-    lev[g] = l;
-    nlev = std::max(nlev, l + 1);
-  }
-  std::vector<int32_t> list;
-  std::vector<int64_t> off;
-  by_level(lev, nlev, list, off);
-  // columns per lane for nearly every group (19 of 20), at most 5
-  int64_t over[2] = {0, 0};
-  for (int64_t g = 0; g < ng; ++g)
-    for (int q = 0; q < 2; ++q) over[q] += ptr[first[g] + 1] - ptr[first[g]] > SWG * (2 + q);
-  const int NC = 20 * over[0] <= ng ? 2 : 20 * over[1] <= ng ? 3 : 5;
-  // a level's groups in order over the slots of its rounds
-  std::vector<int32_t> slot_group, slot_of(ng);
-  std::vector<uint32_t> words;
-  for (int32_t l = 0; l < nlev; ++l) {
-    int64_t oldest = INT64_MAX;  // round of the oldest value the level reads
-    for (int64_t q = off[l]; q < off[l + 1]; ++q) {
-      const int32_t g = list[q];
-      slot_of[g] = static_cast<int32_t>(slot_group.size());
-      slot_group.push_back(g);
-      const int64_t f = first[g], k = ptr[f + 1] - ptr[f];
-      words.push_back(slot_word(f, cnt[g], k > SWG * NC ? SW_TAIL : 0));
-      for (int64_t p = ptr[f]; p < ptr[f + 1]; ++p) oldest = std::min<int64_t>(oldest, slot_of[group_of[idx[p]]] / SWS);
-    }
-    while (slot_group.size() % SWS) {
-      slot_group.push_back(-1);
-      words.push_back(0);
-    }
-    // the level's own values must not reach the ring place of one it reads
-    const int64_t end = static_cast<int64_t>(slot_group.size()) / SWS;
-    if (oldest != INT64_MAX && end - 1 - oldest > ring_rounds(R) - 1) return S;
-    for (size_t q = slot_group.size() - SWS; q < slot_group.size(); ++q) words[q] |= SW_LAST;
-  }
-  S.rounds = (static_cast<int64_t>(slot_group.size()) / SWS + SWD - 1) / SWD * SWD;
-  // the tail loops of the sweep index rounds in 32 bits
-  if ((S.rounds + SWD) * SWS >= (int64_t(1) << 31) || !sweep_pays(nlev, S.rounds, R, NC)) return S;
-  S.word0.assign(static_cast<size_t>(SWD) * SWS, 0);
-  for (size_t q = 0; q < S.word0.size() && q < words.size(); ++q) S.word0[q] = words[q];
-  S.R = R;
-  S.NC = NC;
-  S.levels = nlev;
-  auto fill = [&](auto f) { f(S, ptr, idx, src, dir, first, cnt, slot_group, slot_of, group_of, words); };
-  switch (10 * R + NC) {
-    case 12: fill(fill_records<1, 2>); break;
-    case 13: fill(fill_records<1, 3>); break;
-    case 15: fill(fill_records<1, 5>); break;
-    case 22: fill(fill_records<2, 2>); break;
-    case 23: fill(fill_records<2, 3>); break;
-    case 25: fill(fill_records<2, 5>); break;
-    case 32: fill(fill_records<3, 2>); break;
-    case 33: fill(fill_records<3, 3>); break;
-    default: fill(fill_records<3, 5>); break;
-  }
-  return S;
+  if (R == 1) nc(std::integral_constant<int, 1>());
+  else if (R == 2) nc(std::integral_constant<int, 2>());
+  else nc(std::integral_constant<int, 3>());
 }
 
 class Ic0Impl final : public Ic0Gpu {
@@ -615,11 +430,13 @@ class Ic0Impl final : public Ic0Gpu {
  private:
   struct Sweep {
     int R = 0, NC = 0, rounds = 0;
-    Dev<uint32_t> word0;
-    Dev<int32_t> rec, tptr, tcol;
+    Dev<uint32_t> words;
+    Dev<int32_t> tptr, tcol;
+    Dev<v4i> rec;
     Dev<double> tval;
   };
-  void make_sweep(Sweep& w, const SweepPlan& S);
+  template <int DIR>
+  void make_sweep(Sweep& w, const SweepPlan& S, const int64_t* ptr, const int32_t* idx, const int64_t* map);
   template <int DIR>
   void launch_sweep(const Sweep& w, const double* rin, double* out, const int32_t* done);
 
@@ -663,41 +480,21 @@ Ic0Impl::Ic0Impl(const Csr& a, hipStream_t s) : n_(a.nrows), s_(s) {
       throw std::runtime_error("IC(0): a row of L holds more than " + std::to_string(IC0_MAX_ROW) + " entries");
   }
   const int64_t nnz = lptr[n];
-  // forward levels: 1 + the highest level of the row's columns
-  std::vector<int32_t> lev(n, 0);
-  int32_t nf = n ? 1 : 0;
-  for (int64_t i = 0; i < n; ++i) {
-    int32_t l = 0;
-    for (int64_t p = lptr[i]; p < lptr[i + 1]; ++p) l = std::max(l, lev[lidx[p]] + 1);
-    lev[i] = l;
-    nf = std::max(nf, l + 1);
-  }
-  std::vector<int32_t> flist, blist;
-  by_level(lev, nf, flist, foff_);
-  // U = L^T row-wise (columns increasing) and the map into L's values
-  std::vector<int64_t> uptr(n + 1, 0), tmap(nnz);
-  std::vector<int32_t> uidx(nnz);
-  for (int64_t p = 0; p < nnz; ++p) ++uptr[lidx[p] + 1];
-  for (int64_t j = 0; j < n; ++j) uptr[j + 1] += uptr[j];
-  {
-    std::vector<int64_t> pos(uptr.begin(), uptr.end() - 1);
-    for (int64_t i = 0; i < n; ++i)
-      for (int64_t p = lptr[i]; p < lptr[i + 1]; ++p) {
-        const int64_t q = pos[lidx[p]]++;
-        uidx[q] = static_cast<int32_t>(i);
-        tmap[q] = p;
-      }
-  }
-  // backward levels on U: row j needs the rows i > j of its pattern
-  std::vector<int32_t> blev(n, 0);
-  int32_t nbk = n ? 1 : 0;
-  for (int64_t j = n - 1; j >= 0; --j) {
-    int32_t l = 0;
-    for (int64_t q = uptr[j]; q < uptr[j + 1]; ++q) l = std::max(l, blev[uidx[q]] + 1);
-    blev[j] = l;
-    nbk = std::max(nbk, l + 1);
-  }
-  by_level(blev, nbk, blist, boff_);
+  // the rows' levels, U = L^T row-wise and the map into L's values; the
+  // one-workgroup sweeps where they pay are planned beside the factorization
+  const char* env = std::getenv("RUSTYFEM_IC0_LEVELS");
+  const bool plan = n && !(env && *env && *env != '0');
+  std::vector<int32_t> flist, blist, uidx;
+  std::vector<int64_t> uptr, tmap;
+  std::future<SweepPlan> fplan, bplan;  // (after what they read: destroyed before it)
+  int32_t count = 0;
+  std::vector<int32_t> lev = row_levels(n, lptr, lidx, 1, count);
+  if (plan) fplan = std::async([&, count] { return plan_sweep(n, lptr, lidx, count, 1); });
+  by_level(lev, count, flist, foff_);
+  transpose_pattern(n, lptr, lidx, uptr, uidx, tmap);
+  lev = row_levels(n, uptr, uidx, -1, count);
+  if (plan) bplan = std::async([&, count] { return plan_sweep(n, uptr, uidx, count, -1); });
+  by_level(lev, count, blist, boff_);
 
   lptr_.put(lptr);
   lidx_.put(lidx);
@@ -728,22 +525,22 @@ Ic0Impl::Ic0Impl(const Csr& a, hipStream_t s) : n_(a.nrows), s_(s) {
     shift = shift == 0.0 ? 1e-3 : shift * 4.0;
   }
   shift_ = shift;
-  const char* env = std::getenv("RUSTYFEM_IC0_LEVELS");
-  if (n && !(env && *env && *env != '0')) {
-    // the one-workgroup sweeps where they pay (sweep_pays)
-    const SweepPlan f = plan_sweep(n, lptr, lidx, nullptr, 1);
-    if (f.R) {
-      const SweepPlan b = plan_sweep(n, uptr, uidx, &tmap, -1);
-      if (b.R) {
-        make_sweep(fw_, f);
-        make_sweep(bw_, b);
-      }
-    }
+  uptr_.put(uptr);
+  uidx_.put(uidx);
+  tmap_.put(tmap);
+  SweepPlan fw, bw;
+  if (plan) {
+    fw = fplan.get();
+    bw = bplan.get();
   }
-  if (!bw_.R) {
-    uptr_.put(uptr);
-    uidx_.put(uidx);
-    tmap_.put(tmap);
+  if (fw.R && bw.R) {
+    make_sweep<1>(fw_, fw, lptr_.p, lidx_.p, nullptr);
+    make_sweep<-1>(bw_, bw, uptr_.p, uidx_.p, tmap_.p);
+    // only the launches per level read these
+    uptr_.free();
+    uidx_.free();
+    tmap_.free();
+  } else {
     blist_.put(blist);
     uval_.alloc(nnz);
     if (nnz) {
@@ -756,30 +553,22 @@ Ic0Impl::Ic0Impl(const Csr& a, hipStream_t s) : n_(a.nrows), s_(s) {
   factor_ms_ = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
-void Ic0Impl::make_sweep(Sweep& w, const SweepPlan& S) {
-  w.word0.put(S.word0);
-  w.rec.put(S.rec);
+template <int DIR>
+void Ic0Impl::make_sweep(Sweep& w, const SweepPlan& S, const int64_t* ptr, const int32_t* idx, const int64_t* map) {
+  const int64_t slots = (S.rounds + SWD) * SWS;
+  Dev<int32_t> ring;
+  ring.put(S.ring);
+  w.words.put(S.words);
   w.tptr.put(S.tptr);
-  w.tcol.put(S.tcol);
-  Dev<int32_t> vmap;
-  Dev<int64_t> place, tmap;
-  Dev<SweepCoef> coef;
-  vmap.put(S.vmap);
-  place.put(S.place);
-  coef.put(S.coef);
-  tmap.put(std::vector<int64_t>(S.tmap.begin(), S.tmap.end()));
-  w.tval.alloc(S.tmap.size());
-  double* rec = reinterpret_cast<double*>(w.rec.p);
-  auto blocks = [](size_t c) { return static_cast<unsigned>((c + TB - 1) / TB); };
-  if (!S.vmap.empty())
-    k_ic0_records<<<blocks(S.vmap.size()), TB, 0, s_>>>(static_cast<int64_t>(S.vmap.size()), vmap.p, place.p, lval_.p, rec);
-  if (!S.coef.empty())
-    k_ic0_coefs<<<blocks(S.coef.size()), TB, 0, s_>>>(static_cast<int64_t>(S.coef.size()), coef.p, lval_.p, rec);
-  if (!S.tmap.empty())
-    k_gather<<<std::min(1024u, blocks(S.tmap.size())), TB, 0, s_>>>(static_cast<int64_t>(S.tmap.size()), tmap.p, lval_.p,
-                                                                   w.tval.p);
+  w.tcol.alloc(S.tptr.back());
+  w.tval.alloc(static_cast<size_t>(S.tptr.back()) * S.R);
+  w.rec.alloc(static_cast<size_t>(slots * SWG * record_granules(S.R, S.NC)));
+  with_constants(S.R, S.NC, [&](auto r, auto nc) {
+    k_ic0_records<r(), nc(), DIR><<<static_cast<unsigned>((slots * SWG + TB - 1) / TB), TB, 0, s_>>>(
+        slots, w.words.p, ring.p, w.tptr.p, ptr, idx, map, lval_.p, w.rec.p, w.tcol.p, w.tval.p);
+  });
   ICHK(hipGetLastError());
-  ICHK(hipStreamSynchronize(s_));  // the maps live until here
+  ICHK(hipStreamSynchronize(s_));  // the ring places live until here
   w.rounds = static_cast<int>(S.rounds);
   w.R = S.R;
   w.NC = S.NC;
@@ -787,21 +576,10 @@ void Ic0Impl::make_sweep(Sweep& w, const SweepPlan& S) {
 
 template <int DIR>
 void Ic0Impl::launch_sweep(const Sweep& w, const double* rin, double* out, const int32_t* done) {
-  auto go = [&](auto kernel) {
-    kernel<<<1, SWT, 0, s_>>>(w.rounds, w.word0.p, reinterpret_cast<const v4i*>(w.rec.p), w.tptr.p, w.tcol.p, w.tval.p,
-                              rin, out, done);
-  };
-  switch (10 * w.R + w.NC) {
-    case 12: go(k_ic0_sweep<1, 2, DIR>); break;
-    case 13: go(k_ic0_sweep<1, 3, DIR>); break;
-    case 15: go(k_ic0_sweep<1, 5, DIR>); break;
-    case 22: go(k_ic0_sweep<2, 2, DIR>); break;
-    case 23: go(k_ic0_sweep<2, 3, DIR>); break;
-    case 25: go(k_ic0_sweep<2, 5, DIR>); break;
-    case 32: go(k_ic0_sweep<3, 2, DIR>); break;
-    case 33: go(k_ic0_sweep<3, 3, DIR>); break;
-    default: go(k_ic0_sweep<3, 5, DIR>); break;
-  }
+  with_constants(w.R, w.NC, [&](auto r, auto nc) {
+    k_ic0_sweep<r(), nc(), DIR><<<1, SWT, 0, s_>>>(w.rounds, w.words.p, w.rec.p, w.tptr.p, w.tcol.p, w.tval.p, rin, out,
+                                                   done);
+  });
 }
 
 void Ic0Impl::apply(const double* r, double* z, const int32_t* done) {
