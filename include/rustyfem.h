@@ -380,6 +380,22 @@ int32_t rustyfem_check_plan(size_t n, size_t nn, const int64_t *loc, const doubl
                             const int64_t *indices, const double *data, int32_t leaf, int32_t plant, char *msg,
                             size_t msg_len);
 
+/* Schedule of the IC(0) application for the pattern of a lower triangle (CSC,
+ * rows sorted; additive, host only).  out receives eight values for the
+ * forward and eight for the backward substitution: [0] the rows per group of
+ * the one-workgroup sweep, 0 where every level of rows is a launch (the
+ * application takes sweeps only where both directions have one), [1] its
+ * columns per lane, [2] levels of groups, [3] rounds, [4] the most rounds
+ * between a level's last one and a value that it reads, [5] the bytes it
+ * streams, [6] levels of rows, [7] the rounds that its LDS ring holds.
+ * Returns 0 when every value is read after it is written and before its ring
+ * place is reused, 1 with a description in msg otherwise, -1 on an internal
+ * error.  plant = 1 joins the first two levels, plant = 2 exchanges the ring
+ * places of two rows, so that tests can check that the check fires; plant = 0
+ * checks the real schedule. */
+int32_t rustyfem_sweep_plan(size_t n, const int64_t *colptr, const int64_t *rowidx, int32_t plant, int64_t *out,
+                          char *msg, size_t msg_len);
+
 /* ------------------------------------------------------------ assembly */
 /* Element assembly of linear elastic stiffness matrices on the GPU
  * (additive): replaces the element loop and the serial SystemMatrix::add

@@ -23,6 +23,7 @@
 #include "assembly.hpp"
 #include "eigen.hpp"
 #include "gpu.hpp"
+#include "ic0_plan.hpp"
 #include "indef.hpp"
 #include "mf.hpp"
 #include "mpnn_train.hpp"
@@ -1248,6 +1249,63 @@ int32_t rustyfem_check_plan(size_t n, size_t nn, const int64_t* loc, const doubl
     if (!h) throw std::runtime_error("input rejected before the factorization");
     rf::Plan plan = rf::build_plan(*h->sym, h->colptr, h->rowidx);
     const std::string r = rf::check_plan(plan, plant);
+    if (msg && msg_len) {
+      std::strncpy(msg, r.c_str(), msg_len - 1);
+      msg[msg_len - 1] = 0;
+    }
+    return r.empty() ? 0 : 1;
+  } catch (const std::exception& ex) {
+    set_error(ex.what());
+  } catch (...) {
+    set_error("unknown error");
+  }
+  return -1;
+}
+
+int32_t rustyfem_sweep_plan(size_t n, const int64_t* colptr, const int64_t* rowidx, int32_t plant, int64_t* out, char* msg,
+                          size_t msg_len) {
+  set_error("");
+  try {
+    const int64_t nl = static_cast<int64_t>(n);
+    if (nl >= (int64_t(1) << 31)) throw std::runtime_error("IC(0): too many rows");
+    // U row by row is the strictly lower part column by column
+    std::vector<int64_t> ptr[2], map;
+    std::vector<int32_t> idx[2];
+    ptr[1].assign(n + 1, 0);
+    for (int64_t c = 0; c < nl; ++c) {
+      for (int64_t p = colptr[c]; p < colptr[c + 1]; ++p) {
+        if (rowidx[p] < c || rowidx[p] >= nl || (p > colptr[c] && rowidx[p] <= rowidx[p - 1]))
+          throw std::runtime_error("IC(0): columns of the lower triangle must be sorted without duplicates");
+        if (rowidx[p] > c) idx[1].push_back(static_cast<int32_t>(rowidx[p]));
+      }
+      ptr[1][c + 1] = static_cast<int64_t>(idx[1].size());
+    }
+    rf::transpose_pattern(nl, ptr[1], idx[1], ptr[0], idx[0], map);
+    std::string r;
+    for (int t = 0; t < 2; ++t) {
+      const int dir = t == 0 ? 1 : -1;
+      int32_t levels = 0;
+      rf::row_levels(nl, ptr[t], idx[t], dir, levels);
+      rf::SweepPlan S = rf::plan_sweep(nl, ptr[t], idx[t], levels, dir);
+      int64_t* o = out + 8 * t;
+      o[0] = S.R;
+      o[1] = S.NC;
+      o[2] = S.levels;
+      o[3] = S.rounds;
+      o[4] = S.reach;
+      o[5] = S.R ? S.bytes : 0;
+      o[6] = levels;
+      o[7] = S.R ? rf::ring_rounds(S.R) : 0;
+      if (!S.R) continue;
+      if (plant == 1)
+        for (size_t q = 0; q < S.words.size(); ++q)
+          if (S.words[q] & rf::SW_LAST) {
+            for (int z = 0; z < rf::SWS; ++z) S.words[q + z] &= ~rf::SW_LAST;
+            break;
+          }
+      if (plant == 2) std::swap(S.ring[0], S.ring[nl - 1]);
+      if (r.empty()) r = rf::check_sweep(S, nl, ptr[t], idx[t], dir);
+    }
     if (msg && msg_len) {
       std::strncpy(msg, r.c_str(), msg_len - 1);
       msg[msg_len - 1] = 0;

@@ -61,6 +61,16 @@ bool sweep_pays(int64_t levels, int64_t rounds, int R, int NC) {
          3.4 * R * static_cast<double>(levels);
 }
 
+// Every round streams full records for its 64 slots (16 to 90 KB), also where
+// its level holds one group: a chain of 10^6 rows would take 16 GB for 12 MB of
+// factor.  A sweep may take 16 times the factor instead (a level of five groups
+// on average, whatever the size), or 256 MB, one thousandth of the memory: a
+// chain of up to 15,000 rows (10,000: 9.4 ms an application, 74.6 with a launch
+// per level).
+double stream_limit(int64_t n, int64_t nnz) {
+  return 256e6 + 16.0 * (12.0 * static_cast<double>(nnz) + 16.0 * static_cast<double>(n));
+}
+
 // groups: consecutive rows (in elimination order) whose columns are the first
 // row's columns and the rows of the group before them; first row and rows of
 // every group
@@ -116,7 +126,7 @@ SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vect
   for (int64_t g = 0; g < ng; ++g)
     for (int c = 0; c < cnt[g]; ++c) group_of[first[g] + dir * c] = static_cast<int32_t>(g);
   int32_t nlev = ng ? 1 : 0;
-  int64_t over[2] = {0, 0};
+  int64_t over[2] = {0, 0}, beyond[3] = {0, 0, 0};  // groups of more columns than 2, 3; columns beyond 2, 3, 5
   for (int64_t g = 0; g < ng; ++g) {
     int32_t l = 0;
     const int64_t k = ptr[first[g] + 1] - ptr[first[g]];
@@ -124,6 +134,7 @@ SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vect
     lev[g] = l;
     nlev = std::max(nlev, l + 1);
     for (int q = 0; q < 2; ++q) over[q] += k > SWG * (2 + q);
+    for (int q = 0; q < 3; ++q) beyond[q] += std::max<int64_t>(0, k - SWG * (q == 2 ? 5 : 2 + q));
   }
   std::vector<int32_t> list;
   std::vector<int64_t> off;
@@ -133,12 +144,15 @@ SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vect
   int64_t rounds = 0;
   for (int32_t l = 0; l < nlev; ++l) rounds += (off[l + 1] - off[l] + SWS - 1) / SWS;
   rounds = (rounds + SWD - 1) / SWD * SWD;
+  const int64_t tails = beyond[NC == 5 ? 2 : NC - 2];
+  S.bytes = (rounds + SWD) * SWT * record_granules(R, NC) * 16 + tails * (4 + 8 * R);
+  if (static_cast<double>(S.bytes) > stream_limit(n, static_cast<int64_t>(idx.size()))) return S;
   // the tail loops of the sweep index rounds in 32 bits
   if ((rounds + SWD) * SWS >= (int64_t(1) << 31) || !sweep_pays(nlev, rounds, R, NC)) return S;
   // a level's groups in order over the slots of its rounds
   std::vector<uint32_t> words(static_cast<size_t>((rounds + 2 * SWD) * SWS), 0);
   std::vector<int32_t> ring(n), round_of(ng);
-  int64_t round = 0, tails = 0;
+  int64_t round = 0;
   for (int32_t l = 0; l < nlev; ++l) {
     const int64_t count = off[l + 1] - off[l], end = round + (count + SWS - 1) / SWS;
     int64_t oldest = INT64_MAX;  // round of the oldest value the level reads
@@ -150,7 +164,6 @@ SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vect
       const int64_t at = (slot / SWS % ring_rounds(R)) * (SWS * R) + (slot % SWS) * R;
       for (int c = 0; c < cnt[g]; ++c) ring[f + dir * c] = static_cast<int32_t>(at + c) * 8;
       for (int64_t p = ptr[f]; p < ptr[f + 1]; ++p) oldest = std::min<int64_t>(oldest, round_of[group_of[idx[p]]]);
-      tails += std::max<int64_t>(0, k - SWG * NC);
     }
     // the level's own values must not reach the ring place of one it reads
     if (oldest != INT64_MAX) S.reach = std::max(S.reach, end - 1 - oldest);
@@ -169,10 +182,62 @@ SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vect
   S.NC = NC;
   S.levels = nlev;
   S.rounds = rounds;
-  S.bytes = (rounds + SWD) * SWT * record_granules(R, NC) * 16 + tails * (4 + 8 * R);
   S.words = std::move(words);
   S.ring = std::move(ring);
   return S;
+}
+
+std::string check_sweep(const SweepPlan& S, int64_t n, const std::vector<int64_t>& ptr, const std::vector<int32_t>& idx,
+                        int dir) {
+  const int per = SWS * S.R, places = ring_rounds(S.R) * per;
+  std::vector<int32_t> owner(places, -1);
+  std::vector<uint8_t> seen(n, 0);
+  int64_t rows = 0, levels = 0, tails = 0;
+  if (S.words.size() != static_cast<size_t>((S.rounds + 2 * SWD) * SWS) || S.rounds % SWD) return "rounds";
+  for (int64_t r0 = 0; r0 < S.rounds;) {
+    int64_t r1 = r0;
+    while (r1 < S.rounds && !(S.words[r1 * SWS] & SW_LAST)) ++r1;
+    if (r1 == S.rounds) break;  // the empty rounds at the end
+    ++r1;
+    ++levels;
+    for (int64_t q = r0 * SWS; q < r1 * SWS; ++q) {
+      const uint32_t w = S.words[q];
+      if (((w & SW_LAST) != 0) != (q >= (r1 - 1) * SWS)) return "a round's slots disagree on the level's end";
+      for (int c = 0; c < slot_rows(w); ++c) {
+        const int64_t row = slot_row(w) + dir * c;
+        const int64_t at = (q / SWS % ring_rounds(S.R)) * per + (q % SWS) * S.R + c;
+        if (c >= S.R || row < 0 || row >= n || seen[row]) return "a row is out of range or taken twice";
+        if (S.ring[row] != at * 8) return "a row's ring place is not its slot's";
+        seen[row] = 1;
+        owner[at] = static_cast<int32_t>(row);
+        ++rows;
+      }
+    }
+    for (int64_t q = r0 * SWS; q < r1 * SWS; ++q) {
+      const uint32_t w = S.words[q];
+      if (!slot_rows(w)) continue;
+      const int64_t f = slot_row(w), k = ptr[f + 1] - ptr[f];
+      if (((w & SW_TAIL) != 0) != (k > SWG * S.NC)) return "the tail flag does not fit the row";
+      if (S.tptr[q] != tails) return "the tails overlap";
+      if (w & SW_TAIL) tails += k - SWG * S.NC;
+      for (int c = 0; c < slot_rows(w); ++c) {
+        const int64_t p = ptr[f + dir * c] + (dir > 0 ? 0 : c), o = ptr[f + dir * c] + (dir > 0 ? k : 0);
+        if (ptr[f + dir * c + 1] - ptr[f + dir * c] != k + c || !std::equal(idx.data() + p, idx.data() + p + k, idx.data() + ptr[f]))
+          return "a group's rows differ in their columns";
+        for (int u = 0; u < c; ++u)
+          if (idx[o + u] != (dir > 0 ? f + u : f - c + 1 + u)) return "a group's triangle is not full";
+      }
+      for (int64_t p = ptr[f]; p < ptr[f] + k; ++p) {
+        if (owner[S.ring[idx[p]] / 8] != idx[p]) return "a value is read before it is written or after its place was reused";
+        if (seen[idx[p]] == 1) return "a level reads its own value";
+      }
+    }
+    // 2: of an earlier level
+    for (int64_t q = r0 * SWS; q < r1 * SWS; ++q)
+      for (int c = 0; c < slot_rows(S.words[q]); ++c) seen[slot_row(S.words[q]) + dir * c] = 2;
+    r0 = r1;
+  }
+  return rows == n && levels == S.levels ? "" : "rows or levels are missing";
 }
 
 }  // namespace rf

@@ -2,6 +2,7 @@
 // which round and slot of the one-workgroup sweep every group is taken.
 #pragma once
 #include <cstdint>
+#include <string>
 #include <vector>
 
 namespace rf {
@@ -62,7 +63,8 @@ struct SweepPlan {
 };
 
 // levels: those of the single rows (a launch each without the sweep).  The
-// plan's R is 0 where a sweep is not possible or would not pay.
+// plan's R is 0 where a sweep is not possible, would not pay or would stream
+// more than a small multiple of the factor.
 SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vector<int32_t>& idx, int64_t levels,
                      int dir);
 
@@ -77,5 +79,13 @@ void transpose_pattern(int64_t n, const std::vector<int64_t>& lptr, const std::v
 // rows grouped by level: list (rows in increasing order within a level) and
 // the level offsets
 void by_level(const std::vector<int32_t>& lev, int32_t nlev, std::vector<int32_t>& list, std::vector<int64_t>& off);
+
+// Static check of a plan with R > 0 against its triangle: every row is taken
+// once, by a group whose columns it shares; what a level reads was written by
+// an earlier level and is still in the ring once everything that the level
+// writes has been written (its waves are not held together).  Empty when
+// sound.
+std::string check_sweep(const SweepPlan& S, int64_t n, const std::vector<int64_t>& ptr, const std::vector<int32_t>& idx,
+                        int dir);
 
 }  // namespace rf

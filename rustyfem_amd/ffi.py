@@ -20,7 +20,7 @@ LIB_PATH = os.path.join(HERE, "librustyfem_ffi.so")
 EXPORTS = ["rustyfem_factor", "rustyfem_factor_indef", "rustyfem_factor_unsym", "rustyfem_inertia",
            "rustyfem_solve", "rustyfem_info", "rustyfem_order", "rustyfem_free", "rustyfem_factor_ex",
            "rustyfem_refactor", "rustyfem_solve_device", "rustyfem_solve_device_noalloc", "rustyfem_stats", "rustyfem_last_error", "rustyfem_analyse",
-           "rustyfem_check_plan", "rustyfem_pivots", "rustyfem_factor_stats", "rustyfem_pcg_setup",
+           "rustyfem_check_plan", "rustyfem_sweep_plan", "rustyfem_pivots", "rustyfem_factor_stats", "rustyfem_pcg_setup",
            "rustyfem_pcg_solve", "rustyfem_pcg_stats", "rustyfem_pcg_free", "rustyfem_solve_lower",
            "rustyfem_factor_batch", "rustyfem_refactor_batch", "rustyfem_solve_batch", "rustyfem_solve_batch_device",
            "rustyfem_batch_info", "rustyfem_batch_stats", "rustyfem_batch_order", "rustyfem_free_batch",
@@ -93,6 +93,8 @@ def lib():
         L.rustyfem_analyse.argtypes = fac + [C.c_int32, vp, vp, i64p]
         L.rustyfem_check_plan.restype = C.c_int32
         L.rustyfem_check_plan.argtypes = fac + [C.c_int32, C.c_int32, C.c_char_p, sz]
+        L.rustyfem_sweep_plan.restype = C.c_int32
+        L.rustyfem_sweep_plan.argtypes = [sz, vp, vp, C.c_int32, vp, C.c_char_p, sz]
         L.rustyfem_pivots.restype = C.c_int64
         L.rustyfem_pivots.argtypes = [vp, vp, vp, vp, vp]
         L.rustyfem_factor_stats.restype = None
@@ -189,6 +191,21 @@ def check_plan(p, leaf=16, plant=0):
     if rc < 0:
         raise RuntimeError("rustyfem_check_plan failed: " + last_error())
     return buf.value.decode()
+
+
+def ic0_plan(n, colptr, rowidx, plant=0):
+    """Schedule of the IC(0) application for a lower triangle's pattern
+    (rustyfem_sweep_plan, host only): per direction a dict, and what its check
+    found ('' when sound)."""
+    colptr = np.ascontiguousarray(colptr, dtype=np.int64)
+    rowidx = np.ascontiguousarray(rowidx, dtype=np.int64)
+    out = np.zeros(16, dtype=np.int64)
+    buf = C.create_string_buffer(512)
+    rc = lib().rustyfem_sweep_plan(int(n), colptr.ctypes.data, rowidx.ctypes.data, int(plant), out.ctypes.data, buf, 512)
+    if rc < 0:
+        raise RuntimeError("rustyfem_sweep_plan failed: " + last_error())
+    names = ("rows", "columns", "levels", "rounds", "reach", "bytes", "row_levels", "ring")
+    return [dict(zip(names, map(int, o))) for o in out.reshape(2, 8)], buf.value.decode()
 
 
 def _arrays(p):
