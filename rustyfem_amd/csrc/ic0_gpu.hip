@@ -299,13 +299,15 @@ __global__ __launch_bounds__(SWT) void k_ic0_sweep(int rounds, const uint32_t* _
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) a[r] = half_row_sum(a[r]);
-    // a = -t; x_r = t_r + sum_q coef_q t_q
+    // a = -t; x_r = t_r + sum_{q < r} coef_q t_q (not with zeros for the other
+    // q: a row must not receive what is not finite in a later one)
     double x = a[0];
 #pragma unroll
     for (int r = 1; r < R; ++r)
       if (lane == r) x = a[r];
 #pragma unroll
-    for (int q = 0; q + 1 < R; ++q) x = fma(s.d[NC * R + q], a[q], x);
+    for (int q = 0; q + 1 < R; ++q)
+      if (lane > q) x = fma(s.d[NC * R + q], a[q], x);
     x = -x;
     const int cnt = (s.word >> 2) & 3;
     if (lane < cnt) {

@@ -193,7 +193,7 @@ def check_plan(p, leaf=16, plant=0):
     return buf.value.decode()
 
 
-def ic0_plan(n, colptr, rowidx, plant=0):
+def sweep_plan(n, colptr, rowidx, plant=0):
     """Schedule of the IC(0) application for a lower triangle's pattern
     (rustyfem_sweep_plan, host only): per direction a dict, and what its check
     found ('' when sound)."""

@@ -92,6 +92,30 @@ def test_ic0_sweep_matches_launches_per_level(rf, ora, monkeypatch, case):
         assert np.array_equal(s.precondition(r), z)
 
 
+@pytest.mark.parametrize("rows,at", [(2, 1), (3, 1), (3, 2)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_ic0_sweep_spreads_no_further_than_the_rows(rf, monkeypatch, rows, at, bad):
+    """An entry r[at] that is not finite reaches the rows that depend on its row
+    and no other row of its group: row `rows` depends on the first row of the
+    group before it alone; another full group makes groups of `rows` pay."""
+    n = 2 * rows + 1
+    a = np.diag(np.full(n, 4.0))
+    for f in (0, rows + 1):
+        a[f:f + rows, f:f + rows] -= 1.0 - np.eye(rows)
+    a[rows, 0] = a[0, rows] = -1.0
+    low = lower_csc(a)
+    dirs, _ = rf.sweep_plan(n, *low[:2])
+    assert dirs[0]["rows"] == rows and dirs[1]["rows"] > 0
+    s = rf.Pcg(n, *low, kind="ic0")
+    monkeypatch.setenv("RUSTYFEM_IC0_LEVELS", "1")
+    t = rf.Pcg(n, *low, kind="ic0")
+    r = np.arange(1.0, n + 1)
+    r[at] = bad
+    zs, zt = s.precondition(r), t.precondition(r)
+    assert np.isfinite(zt[rows:]).all()
+    assert np.array_equal(np.isfinite(zs), np.isfinite(zt))
+
+
 def test_ic0_kershaw_shift_matches_oracle(rf, ora):
     a = np.array([[3., -2., 0., 2.], [-2., 3., -2., 0.], [0., -2., 3., -2.], [2., 0., -2., 3.]])
     low = lower_csc(a)

@@ -49,22 +49,22 @@ CASES = {"hex3": lambda: meshes.hex_block(3).to_scipy(), "hex18": lambda: meshes
 def test_schedule_is_sound(case):
     low = lower_csc(CASES[case]())
     n = len(low[0]) - 1
-    dirs, what = ffi.ic0_plan(n, *low)
+    dirs, what = ffi.sweep_plan(n, *low)
     assert what == ""
     for d in dirs:
         if d["rows"]:
             assert d["reach"] < d["ring"] and d["row_levels"] >= d["levels"] >= 1 and d["rounds"] >= d["levels"]
     if all(d["rows"] for d in dirs) and n > 1:
-        assert ffi.ic0_plan(n, *low, plant=2)[1] != ""
+        assert ffi.sweep_plan(n, *low, plant=2)[1] != ""
         if dirs[0]["levels"] > 1:
-            assert ffi.ic0_plan(n, *low, plant=1)[1] != ""
+            assert ffi.sweep_plan(n, *low, plant=1)[1] != ""
 
 
 def test_sweeps_are_taken_where_they_were_measured():
     for make, rows in ((lambda: meshes.hex_block(12).to_scipy(), 3), (lambda: chain(1000), 1),
                        (lambda: meshes.plate_cpe4(60, 6, 1e11, 0.3, nrhs=1).to_scipy(), 2)):
         low = lower_csc(make())
-        dirs, what = ffi.ic0_plan(len(low[0]) - 1, *low)
+        dirs, what = ffi.sweep_plan(len(low[0]) - 1, *low)
         assert what == "" and [d["rows"] for d in dirs] == [rows, rows]
 
 
@@ -77,7 +77,7 @@ def test_stream_is_bounded_by_the_factor(case):
          "band": lambda: band(200_000, 2)}[case]()
     low = lower_csc(a)
     n, nnz = len(low[0]) - 1, len(low[1]) - (len(low[0]) - 1)
-    dirs, what = ffi.ic0_plan(n, *low)
+    dirs, what = ffi.sweep_plan(n, *low)
     assert what == ""
     for d in dirs:
         assert d["bytes"] <= 256e6 + 16 * (12 * nnz + 16 * n)
@@ -87,4 +87,4 @@ def test_stream_is_bounded_by_the_factor(case):
 
 def test_unsorted_pattern_is_refused():
     with pytest.raises(RuntimeError):
-        ffi.ic0_plan(2, np.array([0, 2, 3]), np.array([1, 0, 1]))
+        ffi.sweep_plan(2, np.array([0, 2, 3]), np.array([1, 0, 1]))
