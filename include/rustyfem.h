@@ -386,8 +386,8 @@ int32_t rustyfem_check_plan(size_t n, size_t nn, const int64_t *loc, const doubl
  * the one-workgroup sweep, 0 where every level of rows is a launch (the
  * application takes sweeps only where both directions have one), [1] its
  * columns per lane, [2] levels of groups, [3] rounds, [4] the most rounds
- * between a level's last one and a value that it reads, [5] the bytes it
- * streams, [6] levels of rows, [7] the rounds that its LDS ring holds.
+ * between a level's last one and the first of a level that it reads, [5] the
+ * bytes it streams, [6] levels of rows, [7] the rounds that its LDS ring holds.
  * Returns 0 when every value is read after it is written and before its ring
  * place is reused, 1 with a description in msg otherwise, -1 on an internal
  * error.  plant = 1 joins the first two levels, plant = 2 exchanges the ring

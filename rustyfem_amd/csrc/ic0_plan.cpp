@@ -48,17 +48,25 @@ void transpose_pattern(int64_t n, const std::vector<int64_t>& lptr, const std::v
 
 namespace {
 
-// One workgroup's sweep against a launch per row level, measured per
-// application on C3D8 blocks (both sweeps, row levels in brackets):
-//   8^3 (168) 138 against 896 us, 16^3 (336) 319 / 2,205, 24^3 (504) 702 / 4,386,
-//   32^3 (672) 1,383 / 5,258, 40^3 (840) 2,551 / 7,099, 56^3 (1,176) 10,932 / 11,095.
-// That is about 0.2 us per level and 0.9 us per round of 64 groups, 1.7 us per
-// round where the records exceed the Infinity Cache and come from HBM,
-// against 3.4 us per launch (more where a level has thousands of rows).
-bool sweep_pays(int64_t levels, int64_t rounds, int R, int NC) {
-  const double bytes = static_cast<double>(rounds) * SWT * 8 * (NC * R + R + (NC + 1) / 2 + 1);
-  return 0.2 * static_cast<double>(levels) + (bytes < 128e6 ? 0.9 : 1.7) * static_cast<double>(rounds) <
-         3.4 * R * static_cast<double>(levels);
+// One workgroup's sweep against a launch per level of rows: 0.1 us per level,
+// and per round 0.25 us and the load rate of one compute unit for its records
+// (0.065 us per 8 KB granule row; 0.13 from HBM, where the records of a
+// direction and what else the iteration reads exceed the Infinity Cache),
+// against at least 3.4 us per launch.  Measured, both directions together, us:
+//                              rows of a group, columns a lane, row levels, rounds: sweeps / launches
+//   hexahedra 8^3 / 40^3                 3, 5,  168 /  840,   57 / 1209:    142 /  2,450    1,260 /  7,010
+//   hexahedra 48^3 / 56^3                3, 5, 1008 / 1176, 1992 / 3054:  7,090 / 10,930    9,540 / 11,100
+//   tetrahedra 20^3 / 40^3               3, 3,  180 /  360,  168 / 1116:    276 /  1,630    1,380 /  3,040
+//   quadrilaterals 500 x 200 / 800 x 700 2, 2, 1800 / 4400, 2064 / 10026: 2,080 / 16,500   13,200 / 28,300
+//   2D Laplacian 300^2 / 500^2 / 800^2   1, 2,  599 /  999 / 1599, 1716 / 4410 / 10803:
+//                                           1,220 / 3,130 / 11,800         4,300 / 7,790 / 11,200
+//   3D Laplacian 24^3 / 48^3             1, 2,   70 /  142,  255 / 1800:    203 /  1,225      510 /  1,130
+//   chain 1,000 / band of 5,000 rows     1, 2 / 5, 1000 / 5000, 1002 / 5001: 669 / 8,365     7,400 / 37,000
+bool sweep_pays(int64_t row_levels, int64_t levels, int64_t rounds, int R, int NC) {
+  const double granules = static_cast<double>(record_granules(R, NC)), n = static_cast<double>(rounds);
+  const bool cached = n * SWT * 16 * granules < 128e6;
+  return 0.1 * static_cast<double>(levels) + (0.25 + granules * (cached ? 0.065 : 0.13)) * n <
+         3.4 * static_cast<double>(row_levels);
 }
 
 // Every round streams full records for its 64 slots (16 to 90 KB), also where
@@ -119,19 +127,22 @@ SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vect
   }
   if (R == 1 && static_cast<int64_t>(first.size()) != n) groups(n, ptr, idx, dir, 1, first, cnt);
   const int64_t ng = static_cast<int64_t>(first.size());
-  // no more levels than of rows, and full rounds: most of what will not pay
-  // ends here
-  if (!sweep_pays(levels, ng / SWS, R, 2)) return S;
-  std::vector<int32_t> group_of(n), lev(ng, 0);
-  for (int64_t g = 0; g < ng; ++g)
-    for (int c = 0; c < cnt[g]; ++c) group_of[first[g] + dir * c] = static_cast<int32_t>(g);
+  // full rounds alone: most of what will not pay ends here
+  if (!sweep_pays(levels, 0, ng / SWS, R, 2)) return S;
+  std::vector<int32_t> at(n), lev(ng), low(ng);  // per row: its group's level; per group: level, lowest one read
   int32_t nlev = ng ? 1 : 0;
   int64_t over[2] = {0, 0}, beyond[3] = {0, 0, 0};  // groups of more columns than 2, 3; columns beyond 2, 3, 5
   for (int64_t g = 0; g < ng; ++g) {
-    int32_t l = 0;
+    int32_t l = 0, lo = INT32_MAX;
     const int64_t k = ptr[first[g] + 1] - ptr[first[g]];
-    for (int64_t p = ptr[first[g]]; p < ptr[first[g]] + k; ++p) l = std::max(l, lev[group_of[idx[p]]] + 1);
+    for (int64_t p = ptr[first[g]]; p < ptr[first[g]] + k; ++p) {
+      const int32_t c = at[idx[p]];
+      l = std::max(l, c + 1);
+      lo = std::min(lo, c);
+    }
     lev[g] = l;
+    low[g] = lo;
+    for (int c = 0; c < cnt[g]; ++c) at[first[g] + dir * c] = l;
     nlev = std::max(nlev, l + 1);
     for (int q = 0; q < 2; ++q) over[q] += k > SWG * (2 + q);
     for (int q = 0; q < 3; ++q) beyond[q] += std::max<int64_t>(0, k - SWG * (q == 2 ? 5 : 2 + q));
@@ -148,25 +159,27 @@ SweepPlan plan_sweep(int64_t n, const std::vector<int64_t>& ptr, const std::vect
   S.bytes = (rounds + SWD) * SWT * record_granules(R, NC) * 16 + tails * (4 + 8 * R);
   if (static_cast<double>(S.bytes) > stream_limit(n, static_cast<int64_t>(idx.size()))) return S;
   // the tail loops of the sweep index rounds in 32 bits
-  if ((rounds + SWD) * SWS >= (int64_t(1) << 31) || !sweep_pays(nlev, rounds, R, NC)) return S;
+  if ((rounds + SWD) * SWS >= (int64_t(1) << 31) || !sweep_pays(levels, nlev, rounds, R, NC)) return S;
   // a level's groups in order over the slots of its rounds
   std::vector<uint32_t> words(static_cast<size_t>((rounds + 2 * SWD) * SWS), 0);
-  std::vector<int32_t> ring(n), round_of(ng);
+  std::vector<int32_t> ring(n);
+  std::vector<int64_t> start(nlev);  // the levels' first rounds
   int64_t round = 0;
   for (int32_t l = 0; l < nlev; ++l) {
     const int64_t count = off[l + 1] - off[l], end = round + (count + SWS - 1) / SWS;
-    int64_t oldest = INT64_MAX;  // round of the oldest value the level reads
+    start[l] = round;
+    int32_t lo = INT32_MAX;
     for (int64_t q = 0; q < count; ++q) {
       const int32_t g = list[off[l] + q];
-      const int64_t f = first[g], k = ptr[f + 1] - ptr[f], slot = round * SWS + q;
-      round_of[g] = static_cast<int32_t>(slot / SWS);
-      words[slot] = slot_word(f, cnt[g], k > SWG * NC ? SW_TAIL : 0);
-      const int64_t at = (slot / SWS % ring_rounds(R)) * (SWS * R) + (slot % SWS) * R;
-      for (int c = 0; c < cnt[g]; ++c) ring[f + dir * c] = static_cast<int32_t>(at + c) * 8;
-      for (int64_t p = ptr[f]; p < ptr[f + 1]; ++p) oldest = std::min<int64_t>(oldest, round_of[group_of[idx[p]]]);
+      const int64_t f = first[g], slot = round * SWS + q;
+      words[slot] = slot_word(f, cnt[g], ptr[f + 1] - ptr[f] > SWG * NC ? SW_TAIL : 0);
+      const int64_t o = (slot / SWS % ring_rounds(R)) * (SWS * R) + (slot % SWS) * R;
+      for (int c = 0; c < cnt[g]; ++c) ring[f + dir * c] = static_cast<int32_t>(o + c) * 8;
+      lo = std::min(lo, low[g]);
     }
     // the level's own values must not reach the ring place of one it reads
-    if (oldest != INT64_MAX) S.reach = std::max(S.reach, end - 1 - oldest);
+    // (taken as the first of that value's level)
+    if (lo != INT32_MAX) S.reach = std::max(S.reach, end - 1 - start[lo]);
     if (S.reach > ring_rounds(R) - 1) return S;
     for (int64_t q = (end - 1) * SWS; q < end * SWS; ++q) words[q] |= SW_LAST;
     round = end;

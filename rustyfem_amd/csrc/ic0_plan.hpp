@@ -55,7 +55,7 @@ struct SweepPlan {
   int NC = 0;                   // columns per lane in a record (2, 3 or 5)
   int64_t levels = 0;           // of groups
   int64_t rounds = 0;           // a multiple of SWD
-  int64_t reach = 0;            // rounds between a level's last one and the oldest value that it reads
+  int64_t reach = 0;            // most rounds between a level's last one and the first of a level it reads
   int64_t bytes = 0;            // streamed by a sweep: records, tails
   std::vector<uint32_t> words;  // the slots' words, of rounds + 2 SWD rounds
   std::vector<int32_t> ring;    // per row: the byte offset of its value in the ring
