@@ -273,7 +273,10 @@ int64_t rustyfem_pcg_solve(PcgHandle *h, const double *b, double *x, double tol,
  * residual ||b - A x|| / ||b|| of that direct solution (-1 otherwise), [43] 1
  * when the AMG hierarchy was built on the GPU (0: on the host, as with
  * RUSTYFEM_AMG_HOST_SETUP=1 or a matrix row too long for the device setup's
- * LDS tables).  At most 44 entries. */
+ * LDS tables), [44] 1 when IC(0) is applied by one-workgroup sweeps (0: a
+ * launch per level of rows), [45] and [46] the levels of row groups that they
+ * walk forward and backward, [47] the bytes they stream per application.  At
+ * most 48 entries. */
 void rustyfem_pcg_stats(const PcgHandle *h, double *out, size_t len);
 
 /* Host copy of AMG level `level` of a handle set up with

@@ -24,6 +24,11 @@ class Ic0Gpu {
   virtual int64_t backward_levels() const = 0;
   virtual double factor_ms() const = 0;
   virtual int attempts() const = 0;
+  // one-workgroup sweeps (else a launch per level): the levels of groups they
+  // walk and the bytes both directions stream per application (0 without)
+  virtual bool sweeps() const = 0;
+  virtual int64_t sweep_levels(int dir) const = 0;
+  virtual int64_t sweep_bytes() const = 0;
 };
 
 // Factors the full symmetric CSR matrix `a` (rows sorted) on stream s; every

@@ -428,10 +428,14 @@ class Ic0Impl final : public Ic0Gpu {
   int64_t backward_levels() const override { return static_cast<int64_t>(boff_.size()) - 1; }
   double factor_ms() const override { return factor_ms_; }
   int attempts() const override { return attempts_; }
+  bool sweeps() const override { return bw_.R > 0; }
+  int64_t sweep_levels(int dir) const override { return dir > 0 ? fw_.levels : bw_.levels; }
+  int64_t sweep_bytes() const override { return fw_.bytes + bw_.bytes; }
 
  private:
   struct Sweep {
     int R = 0, NC = 0, rounds = 0;
+    int64_t levels = 0, bytes = 0;
     Dev<uint32_t> words;
     Dev<int32_t> tptr, tcol;
     Dev<v4i> rec;
@@ -574,6 +578,8 @@ void Ic0Impl::make_sweep(Sweep& w, const SweepPlan& S, const int64_t* ptr, const
   w.rounds = static_cast<int>(S.rounds);
   w.R = S.R;
   w.NC = S.NC;
+  w.levels = S.levels;
+  w.bytes = S.bytes;
 }
 
 template <int DIR>
@@ -585,7 +591,7 @@ void Ic0Impl::launch_sweep(const Sweep& w, const double* rin, double* out, const
 }
 
 void Ic0Impl::apply(const double* r, double* z, const int32_t* done) {
-  if (bw_.R) {
+  if (sweeps()) {
     launch_sweep<1>(fw_, r, y_.p, done);
     k_ic0_div<<<static_cast<unsigned>((n_ + TB - 1) / TB), TB, 0, s_>>>(n_, d_.p, y_.p, done);
     launch_sweep<-1>(bw_, y_.p, z, done);

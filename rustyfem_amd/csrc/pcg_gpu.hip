@@ -712,7 +712,7 @@ class PcgImpl final : public PcgGpu {
   }
   PcgResult solve(const double* b, double* x, double tol, int64_t maxit, bool on_device) override;
   void stats(double* out, size_t len) const override {
-    std::vector<double> v(40, 0.0);
+    std::vector<double> v(48, 0.0);  // [40..43] are the caller's
     v[0] = setup_ms_;
     v[1] = solve_ms_;
     v[2] = static_cast<double>(sizes_.size());
@@ -727,6 +727,10 @@ class PcgImpl final : public PcgGpu {
       v[21] = static_cast<double>(ic0_->forward_levels());
       v[22] = static_cast<double>(ic0_->backward_levels());
       v[23] = ic0_->attempts();
+      v[44] = ic0_->sweeps() ? 1.0 : 0.0;
+      v[45] = static_cast<double>(ic0_->sweep_levels(1));
+      v[46] = static_cast<double>(ic0_->sweep_levels(-1));
+      v[47] = static_cast<double>(ic0_->sweep_bytes());
     }
     v[24] = fallback_ ? 1.0 : 0.0;
     v[25] = true_rel_;

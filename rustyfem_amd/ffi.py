@@ -453,8 +453,8 @@ class Pcg:
         return out
 
     def stats(self):
-        o = np.zeros(44)
-        lib().rustyfem_pcg_stats(self._h, o.ctypes.data, 44)
+        o = np.zeros(48)
+        lib().rustyfem_pcg_stats(self._h, o.ctypes.data, 48)
         lv = int(o[2])
         return {"setup_ms": o[0], "solve_ms": o[1], "levels": lv, "complexity": o[3], "spmv_ms": o[4],
                 "spmv_bytes": o[5], "coarse": int(o[6]), "iterations": int(o[7]),
@@ -463,7 +463,8 @@ class Pcg:
                 "fallback": bool(o[24]), "true_rel_residual": o[25], "abandoned_iterations": int(o[26]),
                 "learned_sweeps": int(o[27]), "blocks": [int(b) for b in o[28:28 + min(lv, 12)]],
                 "direct_reason": int(o[40]), "last_direct": bool(o[41]), "direct_rel_residual": o[42],
-                "setup_on_device": bool(o[43])}
+                "setup_on_device": bool(o[43]), "ic0_sweeps": bool(o[44]),
+                "ic0_sweep_levels": (int(o[45]), int(o[46])), "ic0_sweep_bytes": int(o[47])}
 
     def precondition(self, r):
         """z = M r, one application of the preconditioner."""

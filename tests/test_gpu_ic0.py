@@ -61,28 +61,59 @@ def random_dense(n):
     return b @ b.T + n * np.eye(n)
 
 
-SWEEPS = {"hex5": lambda: meshes.hex_block(5).to_scipy(),                  # groups of three rows
-          "hex12x3x7": lambda: meshes.hex_block(12, 3, 7).to_scipy(),
-          "plate31x9": lambda: meshes.plate_cpe4(31, 9, 1e11, 0.3, nrhs=1).to_scipy(),  # of two
-          "laplace9": lambda: meshes.laplacian3d(9).to_scipy(),            # of one
-          "one": lambda: np.array([[2.0]]), "diagonal": lambda: np.diag(np.arange(1.0, 130.0)),
-          "dense41": lambda: random_dense(41),    # rows longer than a lane's registers, group of all rows cut
-          "dense100": lambda: random_dense(100),
-          "wide": lambda: first_column(19900),    # the whole ring in use
-          "too_wide": lambda: first_column(20100)}  # a dependency beyond it: launches per level
+def far(dofs, back, n=400):
+    """Node i depends on the nodes i - 1 and i - back: a level per node, a value
+    read `back` rounds after it was written; `dofs` rows per node."""
+    d = sp.diags([4.0, -0.5, -0.5, -0.25, -0.25], [0, -1, 1, -back, back], shape=(n, n))
+    k = np.full((dofs, dofs), 0.2) + np.diag(np.linspace(1.0, 1.5, dofs))
+    return sp.csc_matrix(sp.kron(d, k))
+
+
+# the matrix, and whether both of its sweeps pay
+SWEEPS = {"hex5": (lambda: meshes.hex_block(5).to_scipy(), True),              # groups of three rows
+          "hex12x3x7": (lambda: meshes.hex_block(12, 3, 7).to_scipy(), True),
+          "plate31x9": (lambda: meshes.plate_cpe4(31, 9, 1e11, 0.3, nrhs=1).to_scipy(), True),  # of two
+          "laplace9": (lambda: meshes.laplacian3d(9).to_scipy(), True),        # of one
+          "one": (lambda: np.array([[2.0]]), True), "diagonal": (lambda: np.diag(np.arange(1.0, 130.0)), True),
+          "dense41": (lambda: random_dense(41), True),   # rows longer than a lane's registers, group of all rows cut
+          "dense100": (lambda: random_dense(100), True),
+          "two_levels": (lambda: first_column(19900), False),
+          # more rounds than the ring holds (104, 156 and 312), with and without tails
+          "hex18": (lambda: meshes.hex_block(18).to_scipy(), True),
+          "hex130x1x1": (lambda: meshes.hex_block(130, 1, 1).to_scipy(), True),
+          "tet18": (lambda: meshes.tet_block(18, seed=2).to_scipy(), True),
+          "plate180x20": (lambda: meshes.plate_cpe4(180, 20, 1e11, 0.3, nrhs=1).to_scipy(), True),
+          "chain700": (lambda: sp.diags([-1.0, 2.5, -1.0], [-1, 0, 1], shape=(700, 700)), True),
+          "laplace28": (lambda: meshes.laplacian3d(28).to_scipy(), True),
+          # values as old as the ring allows, and older ones: a launch per level
+          "far3_in": (lambda: far(3, 103), True), "far3_out": (lambda: far(3, 104), False),
+          "far2_in": (lambda: far(2, 155), True), "far2_out": (lambda: far(2, 156), False),
+          "far1_in": (lambda: far(1, 311, 700), True), "far1_out": (lambda: far(1, 312, 700), False)}
 
 
 @pytest.mark.parametrize("case", sorted(SWEEPS))
 def test_ic0_sweep_matches_launches_per_level(rf, ora, monkeypatch, case):
     """The one-workgroup sweeps against one launch per row level and the oracle
     (the same sums in another order: FP64 rounding of at most 1,000 terms)."""
-    a = SWEEPS[case]()
+    make, sweeps = SWEEPS[case]
+    a = make()
     low = lower_csc(a)
     n = len(low[0]) - 1
     print(f"case ic0 sweep {case} n={n}", flush=True)
     s = rf.Pcg(n, *low, kind="ic0")
     monkeypatch.setenv("RUSTYFEM_IC0_LEVELS", "1")
     t = rf.Pcg(n, *low, kind="ic0")
+    dirs, what = rf.sweep_plan(n, *low[:2])
+    assert what == "" and all(d["rows"] for d in dirs) == sweeps
+    st = s.stats()
+    assert st["ic0_sweeps"] == sweeps and not t.stats()["ic0_sweeps"]
+    if sweeps:
+        assert st["ic0_sweep_levels"] == tuple(d["levels"] for d in dirs)
+        assert st["ic0_sweep_bytes"] == sum(d["bytes"] for d in dirs)
+    if case in ("hex18", "hex130x1x1", "tet18", "plate180x20", "chain700", "laplace28"):
+        assert all(d["rounds"] > d["ring"] for d in dirs)
+    if case.endswith("_in"):
+        assert all(d["reach"] == d["ring"] - 1 and d["rows"] == int(case[3]) for d in dirs)
     rng = np.random.default_rng(12)
     for _ in range(2):
         r = rng.standard_normal(n)
