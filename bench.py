@@ -403,6 +403,9 @@ def run_ic0(args):
     apply_ms = (time.perf_counter() - t1) / reps * 1e3
     nnz_l = (len(ri) - p.n)
     apply_bytes = 2 * nnz_l * 12 + 5 * p.n * 8
+    kernel = (f"k_ic0_sweep (one workgroup per direction, {st['ic0_sweep_levels'][0]} levels of row groups; bytes streamed "
+              "with the padded records: streamed_bytes_per_application)" if st["ic0_sweeps"] else
+              "k_ic0_fwd / k_ic0_bwd (one launch per level of rows)")
     out = {"metric": "IC(0)-PCG solve time to ||r||/||b|| <= 1e-10", "value": float(np.median(times)), "unit": "s",
            "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": float(np.median(times)) * 1e3,
            "higher_is_better": False, "scaling": "weak", "vs_baseline": None, "dtype": "fp64", "data": "synthetic",
@@ -413,7 +416,8 @@ def run_ic0(args):
            "roofline": {"bound": "latency", "achieved": apply_bytes / (apply_ms * 1e-3) / 1e9, "peak": PEAK["hbm_gbs"],
                         "unit": "GB/s", "frac": apply_bytes / (apply_ms * 1e-3) / 1e9 / PEAK["hbm_gbs"],
                         "traffic": None,
-                        "kernel": "k_ic0_fwd / k_ic0_bwd (one launch per level; bytes = 2 nnz(L) 12 + 5 n 8 per application)"}}
+                        "algorithmic_bytes_per_application": apply_bytes,
+                        "streamed_bytes_per_application": st["ic0_sweep_bytes"] or None, "kernel": kernel}}
     d_z.free()
     d_x.free()
     d_b.free()
