@@ -190,15 +190,6 @@ __global__ __launch_bounds__(TB) void k_ic0_div(int64_t n, const double* __restr
 
 // ------------------------------------------------------- one-workgroup sweep
 
-// sum over 8 consecutive lanes, in every lane: quad_perm [1,0,3,2], quad_perm
-// [2,3,0,1], row_half_mirror
-__device__ __forceinline__ double half_row_sum(double v) {
-  v += dpp_d<0xB1>(v);
-  v += dpp_d<0x4E>(v);
-  v += dpp_d<0x141>(v);
-  return v;
-}
-
 typedef int32_t v4i __attribute__((ext_vector_type(4)));
 typedef int32_t v2i __attribute__((ext_vector_type(2)));
 typedef double d2 __attribute__((ext_vector_type(2)));
