@@ -423,13 +423,13 @@ void fill_timings(const rf::Timings& t, double* v) {
   v[12] = t.gemm_flops;
   v[13] = t.tune_ms;
   v[14] = t.tuned_launches;
-  v[15] = t.agpr_launches;
+  v[15] = 0.0;  // the count of a kernel of earlier versions
   for (int i = 0; i < 4; ++i) v[16 + i] = t.refine_history[i];
-  v[20] = t.ilv_launches;
+  v[20] = t.tuned_128x64;
   v[21] = t.refine_undone;
   v[22] = t.fell_back;
   v[23] = t.fallback_rel;
-  v[24] = t.q_launches;
+  v[24] = t.tuned_128x128;
   v[25] = t.small_levels;
 }
 

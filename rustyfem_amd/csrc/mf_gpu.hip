@@ -2028,16 +2028,14 @@ class Impl final : public GpuFactor {
       const char* tm = std::getenv("RUSTYFEM_TUNE_MARGIN");
       if (tm && *tm) tune_margin_ = 1.0f - static_cast<float>(std::atof(tm));
       // RUSTYFEM_AUTOTUNE: unset or 1 = time every GEMM tile shape per launch,
-      // 0 = 64 x 64 tiles everywhere, "128x64" and "128x128" = those
-      // everywhere (FP64 has no 128 x 128: 128 x 64).  The names of earlier
-      // kernels still force one shape: "agpr" and "k64" 64 x 64, "ilv"
-      // 128 x 64, "q" 128 x 128.
+      // 0 or "64x64" = 64 x 64 tiles everywhere, "128x64" and "128x128" =
+      // those everywhere (FP64 has no 128 x 128: 128 x 64).
       const char* a = std::getenv("RUSTYFEM_AUTOTUNE");
       auto is = [a](const char* n) { return a && std::strcmp(a, n) == 0; };
-      const int8_t force = is("128x64") || is("ilv") ? GEMM_128x64
-                           : is("128x128") || is("q") ? std::min<int>(GEMM_128x128, kGemmShapes<T> - 1)
-                                                      : GEMM_64x64;
-      autotune_ = !(a && *a == '0') && force == GEMM_64x64 && !is("64x64") && !is("agpr") && !is("k64");
+      const int8_t force = is("128x64")    ? GEMM_128x64
+                           : is("128x128") ? std::min<int>(GEMM_128x128, kGemmShapes<T> - 1)
+                                           : GEMM_64x64;
+      autotune_ = !(a && *a == '0') && force == GEMM_64x64 && !is("64x64");
       gemm_pick_.assign(P_.gemm.size(), force);
       // In a GEMM launch where most tiles update at most 64 rows and columns
       // (small fronts), those tiles go first in its range and run as one
@@ -2627,9 +2625,8 @@ class Impl final : public GpuFactor {
     HIPCHK(hipEventElapsedTime(&ms, e0_, e1_));
     tm_.tune_ms = ms;
     tm_.tuned_launches = static_cast<double>(ph.size());
-    tm_.agpr_launches = 0.0;
-    tm_.ilv_launches = static_cast<double>(count[GEMM_128x64]);
-    tm_.q_launches = NV > GEMM_128x128 ? static_cast<double>(count[NV - 1]) : 0.0;
+    tm_.tuned_128x64 = static_cast<double>(count[GEMM_128x64]);
+    tm_.tuned_128x128 = NV > GEMM_128x128 ? static_cast<double>(count[NV - 1]) : 0.0;
     tuned_ = true;
   }
 

@@ -346,36 +346,29 @@ def test_pivot_steps_at_partial_blocks(rf, monkeypatch, precision, k):
 
 
 @pytest.mark.parametrize("precision", [None, "mixed"])
-def test_gemm_register_layouts_agree(rf, monkeypatch, precision):
-    """The Schur GEMM kernels (k_gemm, k_gemm_agpr, k_gemm_ilv, k_gemm_k64 and,
-    in FP32, k_gemm_q) run the same arithmetic: forcing any one gives
-    identical D and solutions, and the autotuner times every GEMM launch of
-    the plan."""
+def test_gemm_tile_shapes_agree(rf, monkeypatch, precision):
+    """The tile shapes of the Schur GEMM (64 x 64, 128 x 64 and, in FP32,
+    128 x 128) run the same arithmetic: forcing any one for every launch gives
+    the same D and solutions as the autotuned mix, and the autotuner times
+    every GEMM launch of the plan and none where a shape is forced."""
     p = meshes.hex_block(12, nrhs=2, seed=5)
-    monkeypatch.setenv("RUSTYFEM_AUTOTUNE", "0")
-    h_v, _, d_v = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
-    monkeypatch.setenv("RUSTYFEM_AUTOTUNE", "agpr")
-    h_a, _, d_a = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
-    monkeypatch.setenv("RUSTYFEM_AUTOTUNE", "ilv")
-    h_i, _, d_i = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
-    monkeypatch.setenv("RUSTYFEM_AUTOTUNE", "k64")
-    h_k, _, d_k = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
-    monkeypatch.setenv("RUSTYFEM_AUTOTUNE", "q")
-    h_q, _, d_q = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
-    monkeypatch.delenv("RUSTYFEM_AUTOTUNE")
-    h_t, _, d_t = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
-    assert np.array_equal(d_a, d_v) and np.array_equal(d_i, d_v) and np.array_equal(d_k, d_v)
-    assert np.array_equal(d_q, d_v)
-    assert np.array_equal(d_t, d_v)
-    x = h_v.solve(p.rhs)
-    for h in (h_a, h_i, h_k, h_q, h_t):
-        assert np.array_equal(h.solve(p.rhs), x)
-    st = h_t.stats()
+    out = {}
+    for shape in ("64x64", "128x64", "128x128", None):
+        if shape is None:
+            monkeypatch.delenv("RUSTYFEM_AUTOTUNE")
+        else:
+            monkeypatch.setenv("RUSTYFEM_AUTOTUNE", shape)
+        h, _, d = rf.Handle.factor(p, want_d=True, precision=precision, max_refine=0)
+        out[shape] = d, h.solve(p.rhs), h.stats()
+    for shape in ("128x64", "128x128", None):
+        assert np.array_equal(out[shape][0], out["64x64"][0])
+        assert np.array_equal(out[shape][1], out["64x64"][1])
+    st = out.pop(None)[2]
     assert st["tuned_launches"] > 0
-    assert 0 <= st["agpr_launches"] + st["ilv_launches"] + st["q_launches"] <= st["tuned_launches"]
+    assert 0 <= st["ilv_launches"] + st["q_launches"] <= st["tuned_launches"]
     if precision is None:
         assert st["q_launches"] == 0
-    assert h_v.stats()["tuned_launches"] == 0 and h_i.stats()["tuned_launches"] == 0
+    assert all(o[2]["tuned_launches"] == 0 for o in out.values())
 
 
 @pytest.mark.parametrize("k,u", [(3, 1), (7, 65), (17, 129), (63, 64), (65, 127), (130, 200), (520, 193)])
