@@ -21,8 +21,10 @@
 // as one group (up to three rows), which divides the levels by the node's DOF
 // count.  One workgroup walks all levels with the recent values of the
 // solution in LDS (k_ic0_sweep); where the levels are wide enough to feed the
-// whole GPU, or a dependency reaches further back than the LDS ring, every
-// level of rows is a launch (k_ic0_fwd / k_ic0_bwd, 16 lanes per row).
+// whole GPU, a dependency reaches further back than the LDS ring, or the levels
+// are so many and narrow that their padded records outgrow the factor
+// (ic0_plan.cpp), every level of rows is a launch (k_ic0_fwd / k_ic0_bwd, 16
+// lanes per row).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -211,7 +213,7 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 // 20^3 block (26,460 rows, 420 row levels, 140 of groups), per sweep: one
 // launch per row level 1,430 us; columns and values row by row in the
 // factor's order 294-355 us (more loads, selects and address arithmetic); this
-// 194 us (0.9 us per round of 88 KB, 98 GB/s: the rate of one unit's L1).
+// 212 us (1.0 us per round of 88 KB, 92 GB/s: the rate of one unit's L1).
 template <int R, int NC, int DIR>
 __global__ __launch_bounds__(SWT) void k_ic0_sweep(int rounds, const uint32_t* __restrict__ word0,
                                                    const v4i* __restrict__ rec, const int32_t* __restrict__ tptr,
