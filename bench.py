@@ -712,7 +712,7 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py runs on one GPU: the multifrontal factorization of one problem is not sharded "
-              "across GPUs in this build (see DESIGN.md for how it would shard)", file=sys.stderr)
+              "across GPUs in this build", file=sys.stderr)
         sys.exit(2)
     if args.workload == "amg":
         run_amg(args)
