@@ -69,6 +69,14 @@ def far(dofs, back, n=400):
     return sp.csc_matrix(sp.kron(d, k))
 
 
+def band(dofs, width, n=400):
+    """Node i coupled to the `width` nodes before it, `dofs` rows per node."""
+    d = sp.diags([np.full(n, 3.0 * width)] + [np.full(n - q, -1.0 / q) for q in range(1, width + 1)],
+                 list(range(0, -width - 1, -1)), shape=(n, n))
+    d = d + sp.tril(d, -1).T
+    return sp.csc_matrix(sp.kron(d, np.full((dofs, dofs), 0.2) + np.diag(np.linspace(1.0, 1.5, dofs))))
+
+
 # the matrix, and whether both of its sweeps pay
 SWEEPS = {"hex5": (lambda: meshes.hex_block(5).to_scipy(), True),              # groups of three rows
           "hex12x3x7": (lambda: meshes.hex_block(12, 3, 7).to_scipy(), True),
@@ -85,6 +93,11 @@ SWEEPS = {"hex5": (lambda: meshes.hex_block(5).to_scipy(), True),              #
           "plate180x20": (lambda: meshes.plate_cpe4(180, 20, 1e11, 0.3, nrhs=1).to_scipy(), True),
           "chain700": (lambda: sp.diags([-1.0, 2.5, -1.0], [-1, 0, 1], shape=(700, 700)), True),
           "laplace28": (lambda: meshes.laplacian3d(28).to_scipy(), True),
+          # 2, 3 and 5 columns a lane, and columns beyond the record
+          "band1_20": (lambda: band(1, 20), True), "band1_37": (lambda: band(1, 37), True),
+          "band1_60": (lambda: band(1, 60), True), "band2_10": (lambda: band(2, 10), True),
+          "band2_20": (lambda: band(2, 20), True), "band2_30": (lambda: band(2, 30), True),
+          "band3_4": (lambda: band(3, 4), True), "band3_20": (lambda: band(3, 20), True),
           # values as old as the ring allows, and older ones: a launch per level
           "far3_in": (lambda: far(3, 103), True), "far3_out": (lambda: far(3, 104), False),
           "far2_in": (lambda: far(2, 155), True), "far2_out": (lambda: far(2, 156), False),
