@@ -213,7 +213,7 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 // 20^3 block (26,460 rows, 420 row levels, 140 of groups), per sweep: one
 // launch per row level 1,430 us; columns and values row by row in the
 // factor's order 294-355 us (more loads, selects and address arithmetic); this
-// 212 us (1.0 us per round of 88 KB, 92 GB/s: the rate of one unit's L1).
+// 209 us (1.0 us per round of 88 KB, 93 GB/s: the rate of one unit's L1).
 template <int R, int NC, int DIR>
 __global__ __launch_bounds__(SWT) void k_ic0_sweep(int rounds, const uint32_t* __restrict__ word0,
                                                    const v4i* __restrict__ rec, const int32_t* __restrict__ tptr,
@@ -296,11 +296,12 @@ __global__ __launch_bounds__(SWT) void k_ic0_sweep(int rounds, const uint32_t* _
     // q: a row must not receive what is not finite in a later one)
     double x = a[0];
 #pragma unroll
-    for (int r = 1; r < R; ++r)
-      if (lane == r) x = a[r];
+    for (int r = 1; r < R; ++r) {
+      double t = a[r];
 #pragma unroll
-    for (int q = 0; q + 1 < R; ++q)
-      if (lane > q) x = fma(s.d[NC * R + q], a[q], x);
+      for (int q = 0; q < r; ++q) t = fma(s.d[NC * R + q], a[q], t);
+      if (lane == r) x = t;
+    }
     x = -x;
     const int cnt = (s.word >> 2) & 3;
     if (lane < cnt) {
